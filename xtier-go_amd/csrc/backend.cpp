@@ -171,7 +171,10 @@ void Backend::matmul_dev(const xtg_nvfp4* ws, int nw, const void* x, int x_dtype
   const int k = ws[0].k;
   XTG_CHECK(m >= 1 && m <= kMaxDeviceRows, "matmul: %d rows (1..%d per device call)", m, kMaxDeviceRows);
   XTG_CHECK(reinterpret_cast<uintptr_t>(x) % 16 == 0, "matmul: rows at %p are not 16-byte aligned", x);
-  if (m <= kMaxRows) {   // the GEMV takes the rows as they are when its shape allows
+  // up to 8 rows the GEMV takes the rows as they are when its shape allows; more BF16 rows take the GEMM's one-part
+  // operand, exact for them, at half the matrix ops (XTG_GEMM_PARTS chooses between the parts of the other operand)
+  const bool x16 = m > kMaxRows && x_dtype == kXBF16 && !std::getenv("XTG_GEMM_PARTS");
+  if (m <= kMaxRows || x16) {
     XTG_CHECK(x_dtype == kXF32 || x_dtype == kXBF16, "matmul: unknown activation type %d", x_dtype);
     XTG_CHECK(x && y, "matmul: NULL input or output");
     GemvCall c;
@@ -188,6 +191,14 @@ void Backend::matmul_dev(const xtg_nvfp4* ws, int nw, const void* x, int x_dtype
     c.x = x;
     c.x_dtype = x_dtype;
     c.k = k;
+    if (x16) {
+      ensure(op_, op_size_, size_t((m + 15) / 16) * op16_block_bytes(k));
+      timed([&] { return launch_prep_x16(x, m, k, op_, stream_); });
+      c.xop = op_;
+      c.x16 = true;
+      timed([&] { return launch_gemm(c, stream_); });
+      return;
+    }
     if (gemv_takes_raw(c)) {
       timed([&] { return launch_gemv(c, stream_); });
       return;

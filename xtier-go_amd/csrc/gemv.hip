@@ -187,6 +187,61 @@ std::string launch_prep_x(const void* x, int x_dtype, int m, int k, void* op, hi
   return "prep_x_kernel";
 }
 
+// One work-group per BF16 row: the row as one f16 part (prep_x_kernel's scaled high part; the low part of a BF16 value
+// is zero), column j % 16 of its 16-row block. Half of prep_x_kernel's bytes written: 1500 rows of 7168 in 8 us
+// against 14.6.
+__global__ void __launch_bounds__(kPrepThreads) prep_x16_kernel(const void* __restrict__ x, int k, int kt,
+                                                                char* __restrict__ op, size_t stride) {
+  __shared__ float red[2 * kPrepThreads / 64];
+  const int row = blockIdx.x, tid = threadIdx.x, j = row & 15;
+  f16x8* __restrict__ xop = reinterpret_cast<f16x8*>(op + size_t(row >> 4) * stride);
+  const int chunks = kt * 16;
+  float v[kPrepChunks][8];
+  float mx = 0.f;
+#pragma unroll
+  for (int u = 0; u < kPrepChunks; ++u) {
+    const int c = tid + u * kPrepThreads;
+    load_chunk(x, kXBF16, row, k, c < chunks ? c : chunks, v[u]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(v[u][i]));
+  }
+  for (int c = tid + kPrepChunks * kPrepThreads; c < chunks; c += kPrepThreads) {
+    float w[8];
+    load_chunk(x, kXBF16, row, k, c, w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(w[i]));
+  }
+  const int e = operand_exponent(block_max<kPrepThreads>(mx, red));
+  const float up = ldexpf(1.f, e);
+  if (tid == 0) reinterpret_cast<float*>(op + size_t(row >> 4) * stride + size_t(kt) * 4096)[j] = ldexpf(1.f, -e);
+  auto store = [&](int c, const float (&w)[8]) {
+    f16x8 h;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) h[i] = (_Float16)(w[i] * up);
+    const int q = c & 15, g = q >> 2, t = q & 3;
+    xop[(size_t(c >> 4) * 4 + size_t(t)) * 64 + size_t(4 * j + g)] = h;
+  };
+#pragma unroll
+  for (int u = 0; u < kPrepChunks; ++u) {
+    const int c = tid + u * kPrepThreads;
+    if (c < chunks) store(c, v[u]);
+  }
+  for (int c = tid + kPrepChunks * kPrepThreads; c < chunks; c += kPrepThreads) {
+    float w[8];
+    load_chunk(x, kXBF16, row, k, c, w);
+    store(c, w);
+  }
+}
+
+std::string launch_prep_x16(const void* x, int m, int k, void* op, hipStream_t stream) {
+  XTG_CHECK(m >= 1 && k > 0 && k % 16 == 0, "prep_x: %d rows of %d (a multiple of 16)", m, k);
+  XTG_CHECK(reinterpret_cast<uintptr_t>(x) % 16 == 0, "prep_x: activations at %p are not 16-byte aligned", x);
+  hipLaunchKernelGGL(prep_x16_kernel, dim3(unsigned(m)), dim3(kPrepThreads), 0, stream, x, k, (k + kTileK - 1) / kTileK,
+                     static_cast<char*>(op), op16_block_bytes(k));
+  HIP_CHECK(hipGetLastError());
+  return "prep_x16_kernel";
+}
+
 // ------------------------------------------------------------------------------------------------------ GEMV
 
 struct GemvArgs {

@@ -47,6 +47,12 @@ enum XDtype { kXF32 = 0, kXBF16 = 1 };
 std::string launch_prep_x(const void* x, int x_dtype, int m, int k, void* op, hipStream_t stream,
                           float* copy = nullptr);
 
+// BF16 rows for the GEMM: an f16 holds a BF16's 8 significant bits, so one part is exact where the two-part operand
+// is (its low parts would all be zero). Blocks of 16 rows in the layout of an 8-row group, column c = row c's f16
+// (scaled by 2^s_c, s as the two-part operand's), then the 16 row factors 2^-s_c.
+inline size_t op16_block_bytes(int k) { return xop_bytes(k) + 2 * kMaxRows * sizeof(float); }
+std::string launch_prep_x16(const void* x, int m, int k, void* op, hipStream_t stream);
+
 struct GemvCall {
   const PackedNvfp4* w[4] = {nullptr, nullptr, nullptr, nullptr};
   int nw = 0;
@@ -60,6 +66,7 @@ struct GemvCall {
   int x_dtype = 0;
   int k = 0;
   int parts = 2;   // the GEMM's activation parts (prefill chunks): 2, high and low f16; 1, the high part alone
+  bool x16 = false;   // the GEMM's xop is launch_prep_x16's (BF16 rows, one part)
   // the GEMV on a prepared operand (2..8 rows): 2 splits K in two halves whose partial outputs go to y (the first
   // k-tiles) and to y + y_part (the rest), each laid out as y_off says; the consumer adds them, first + second.
   // Each work-group then reads half of the rows' operand (the bytes its k-range needs), the share of a launch that
