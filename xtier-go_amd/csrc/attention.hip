@@ -28,9 +28,9 @@
 //     and the query rows are stacked as MFMA columns (q-col = row * group + head), so every K and V byte is read
 //     once per KV head. Each wave streams its tiles with the next tile's loads in flight; the waves' states are
 //     merged in LDS into one partial per q-col.
-//   Own keys (FP32, not rounded to the cache's BF16), one more partial: for the attention call, FP32 MFMA over
-//     tiles of 16 q-cols x 16 keys (attn_own_mfma_kernel); inside the decode step's producer (qk_produce_kernel),
-//     one wave per q-col on the vector ALUs.
+//   Own keys (FP32, not rounded to the cache's BF16), more partials: for the attention call and prefill chunks,
+//     exact BF16 splits of both operands on the matrix cores (attn_own_kernel); inside the decode step's producer
+//     (qk_produce_kernel), one wave per q-col on the vector ALUs.
 //   attn_merge_kernel / attn_gate_kernel: one work-group per query row merges its partials (kv.cpp:262-285);
 //     the gate variant applies the decode step's sigmoid gate and norm and writes the o-projection's operand.
 #include <algorithm>
@@ -965,17 +965,6 @@ __device__ inline void write_partial(float* acc, float* ml, size_t rec, float M,
   }
 }
 
-// Own keys on the matrix cores (FP32 MFMA 16x16x4), for calls of many rows: one wave per tile of 16 q-cols of a
-// row block and chunk of kOwnChunk keys of the range any of its columns sees (from the range's first key), 16 keys
-// a step; each chunk leaves its own partial record (own-key record `splits + chunk`), an empty chunk the record of
-// no key (max -inf, sum 0), which the merges skip. Chunks put several waves on a SIMD where one wave per column
-// tile had every step wait for its loads.
-//   S^T (16 keys x 16 q-cols) = K Q^T: at step s lane group g (lane / 16) feeds dim (D / 4) g + s of key / q-col
-//   lane % 16, so each lane's K and Q values are D / 4 contiguous floats; lane (g, j) gets S^T[key 4 g + r][col j].
-//   O^T (D x 16 q-cols) += V^T P^T: step r sums keys 4 g + r over the lane groups, so P^T comes straight from the
-//   scores' registers; lane (g, j) holds O^T[16 t + 4 g + r][col j] in accumulator t.
-// The online softmax runs per column over the lane groups (max and sum through two xor shuffles); the partial
-// record (M, L, O) goes to the own-key slot (split index `splits`) of the column's block.
 struct OwnArgs {
   const float* q;          // [n_own][heads][D]
   const float* k;          // [n_own][kv_heads][D]
@@ -983,21 +972,30 @@ struct OwnArgs {
   float* acc;              // partials as ScanArgs
   float* ml;
   size_t blk_records;
-  int b0, nblocks, rpb, n_own, heads, kv_heads, group, window, splits, splits1, qpad, tiles;   // tiles per block
-  int own;                 // key chunks per column tile
+  int b0, nblocks, rpb, n_own, heads, kv_heads, group, window, splits, splits1, qpad;
+  int own, run;            // runs of keys, and keys in each (a multiple of the tile)
   float scale2;
 };
 
+// Own keys on the matrix cores, for calls of few rows (own_few_rows): FP32 MFMA 16x16x4, one wave per tile of 16
+// q-cols of a row block over all the keys that any of its columns sees, 16 keys a step, one record. What bounds such a
+// call is one wave's chain of loads and the code it runs once, so nothing is staged or shared:
+//   S^T (16 keys x 16 q-cols) = K Q^T: at step s lane group g (lane / 16) feeds dim (D / 4) g + s of key / q-col
+//   lane % 16, so each lane's K and Q values are D / 4 contiguous floats; lane (g, j) gets S^T[key 4 g + r][col j].
+//   O^T (D x 16 q-cols) += V^T P^T: step r sums keys 4 g + r over the lane groups, so P^T comes straight from the
+//   scores' registers; lane (g, j) holds O^T[16 t + 4 g + r][col j] in accumulator t.
+// The online softmax runs per column over the lane groups (max and sum through two xor shuffles); the partial
+// record (M, L, O) goes to the own-key slot (split index `splits`) of the column's block.
 template <int D>
 __global__ void __launch_bounds__(256) attn_own_mfma_kernel(const OwnArgs a) {
   constexpr int S = D / 4, T = D / 16;
   const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
   const int w = int(blockIdx.x) * 4 + int(threadIdx.x >> 6);
-  const int per_blk = a.kv_heads * a.tiles * a.own;
+  const int tiles = a.qpad / 16, per_blk = a.kv_heads * tiles;
   if (w >= per_blk * a.nblocks) return;   // no barriers below: a spare wave just leaves
-  // the last (longest) blocks first; a tile's chunks in consecutive waves (one work-group shares its q loads)
-  const int blk = a.b0 + a.nblocks - 1 - w / per_blk, ct = (w % per_blk) / a.own, chunk = w % a.own;
-  const int kvh = ct / a.tiles, tile = ct % a.tiles;
+  // the last (longest) blocks first
+  const int blk = a.b0 + a.nblocks - 1 - w / per_blk, ct = w % per_blk;
+  const int kvh = ct / tiles, tile = ct % tiles;
   const int row0 = blk * a.rpb, n_rows = min(a.rpb, a.n_own - row0), cols = n_rows * a.group;
   const int qc = tile * 16 + j;
   if (tile * 16 >= cols) return;           // a padding tile of the block
@@ -1006,8 +1004,7 @@ __global__ void __launch_bounds__(256) attn_own_mfma_kernel(const OwnArgs a) {
   const int lo = a.window > 0 ? max(0, i - a.window + 1) : 0;
   // the tile's key range: its rows run from the first column's to the last live column's
   const int i_first = row0 + (tile * 16) / a.group, i_last = row0 + (min(tile * 16 + 15, cols - 1)) / a.group;
-  const int k0 = a.window > 0 ? max(0, i_first - a.window + 1) : 0;
-  const int kmin = k0 + chunk * kOwnChunk, kmax = min(i_last + 1, kmin + kOwnChunk);   // this chunk's keys
+  const int kmin = a.window > 0 ? max(0, i_first - a.window + 1) : 0, kmax = i_last + 1;
 
   float qv[S];
   {
@@ -1083,11 +1080,313 @@ __global__ void __launch_bounds__(256) attn_own_mfma_kernel(const OwnArgs a) {
   L += __shfl_xor(L, 16);
   L += __shfl_xor(L, 32);
   if (!live) return;
-  const size_t rec = (size_t(kvh) * size_t(a.splits1) + size_t(a.splits + chunk)) * size_t(a.qpad) + size_t(qc);
+  const size_t rec = (size_t(kvh) * size_t(a.splits1) + size_t(a.splits)) * size_t(a.qpad) + size_t(qc);
   float* acc = a.acc + size_t(blk) * a.blk_records * D + rec * D;
   if (g == 0) *reinterpret_cast<float2*>(a.ml + (size_t(blk) * a.blk_records + rec) * 2) = make_float2(M, L);
 #pragma unroll
   for (int t = 0; t < T; ++t) *reinterpret_cast<f32x4*>(acc + 16 * t + 4 * g) = o[t];
+}
+
+// Own keys on the matrix cores, for calls of many rows. FP32 rows go through v_mfma_f32_16x16x32_bf16 in three exact
+// BF16 terms each (split_exact: 24 bits = 3 x 8): of the nine products of two such values the six down to 2^-16 are
+// taken, what is dropped is below 2^-23 of the product, and sums are FP32. That is 6 matrix ops of 16 cycles for what
+// v_mfma_f32_16x16x4_f32 takes 8 of 32 cycles for.
+//
+// A work-group of 4 waves takes 4 consecutive row blocks (a wave each, its 2 x 16 q-cols) of one KV head and one of
+// `own` runs of keys, in tiles of 32 keys whose K and V the 4 waves share: each wave loads a quarter of a tile as FP32
+// (the next tile's during this tile's math), splits it once and puts the terms into LDS in operand order, K as
+// [16-key block][32-dim chunk][term][lane], V as [16-dim block][term][lane], as the cache holds them. A wave leaves
+// out the tiles that none of its rows sees. A run without a key of the block leaves the record of no key (max -inf,
+// sum 0), which the merges skip.
+// Waves per SIMD: one at 64 and 128 dims and two work-groups a CU; at 256 dims two waves share a row block
+// (own_halves), one work-group a CU. LDS reads take half of the matrix ops' time (each operand read feeds two column
+// blocks: with one a wave they would take all of it). Measured (512 rows, no cached keys, in the kernel): 16 / 4 heads
+// of 256, 107 us with the FP32 kernel, 38 us here; 32 / 8 of 128, 51 and 27 us. The matrix ops are busy for a fifth of
+// that: a run is 3-4 tiles long, each 3-4 us of scores 1.1, softmax and splits 0.7, outputs 1.4 and barriers 0.8 in a
+// chain, after about 4 us of first loads and of code that is fetched the first time.
+
+// x = t0 + t1 + t2 exactly: each term the upper half of what is left (8 bits of the 24). ANY: an infinity or a NaN
+// comes as the last term alone, which meets the other operand's first term only (as the first it would meet second and
+// third terms that are zero, and make NaN of an infinity). Without ANY, x is finite or NaN.
+__device__ inline uint32_t upper_halves(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+template <bool ANY>
+__device__ inline void split_exact(const float (&v)[8], bf16x8 (&t)[3]) {
+  float x[8], r1[8], r2[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bool finite = !ANY || __builtin_fabsf(v[e]) < INFINITY;
+    x[e] = finite ? v[e] : 0.f;
+    r1[e] = x[e] - __uint_as_float(__float_as_uint(x[e]) & 0xffff0000u);
+    r2[e] = r1[e] - __uint_as_float(__float_as_uint(r1[e]) & 0xffff0000u);
+    if (!finite) r2[e] = v[e];
+  }
+  uint4 u[3];
+  u[0] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
+  u[1] = make_uint4(upper_halves(r1[0], r1[1]), upper_halves(r1[2], r1[3]), upper_halves(r1[4], r1[5]),
+                    upper_halves(r1[6], r1[7]));
+  u[2] = make_uint4(upper_halves(r2[0], r2[1]), upper_halves(r2[2], r2[3]), upper_halves(r2[4], r2[5]),
+                    upper_halves(r2[6], r2[7]));
+#pragma unroll
+  for (int n = 0; n < 3; ++n) t[n] = __builtin_bit_cast(bf16x8, u[n]);
+}
+
+// The six products of A = a0 + a1 + a2 and B = b0 + b1 + b2, smallest first, onto one accumulator per column block.
+template <int QB>
+__device__ inline void mfma_split(const bf16x8 (&A)[3], const bf16x8 (&B)[QB][3], f32x4 (&d)[QB]) {
+  constexpr int ta[6] = {2, 1, 0, 1, 0, 0}, tb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+  for (int n = 0; n < 6; ++n)
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) d[qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[ta[n]], B[qb][tb[n]], d[qb], 0, 0, 0);
+}
+
+// The order of N groups of 3 operand reads and M matrix ops: each group's reads go out before the matrix ops of the
+// group before (the compiler by itself waits for a group's reads right before its first matrix op).
+template <int N, int M>
+__device__ __forceinline__ void pace_reads() {
+  __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // LDS reads
+#pragma unroll
+  for (int n = 1; n < N; ++n) {
+    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, M, 0);   // matrix ops
+  }
+  __builtin_amdgcn_sched_group_barrier(0x8, M, 0);
+}
+
+// Waves of a row block: at 256 dims two share its q-cols, each with half of the dims (its half of the score sums,
+// exchanged through LDS, and its half of the outputs), so that two waves fit a SIMD.
+template <int D>
+constexpr int own_halves() { return D == 256 ? 2 : 1; }
+// K and V terms of one tile, and the exchanged score sums (16 floats a lane).
+template <int D>
+constexpr size_t own_lds_bytes() {
+  return size_t(2 * kTile) * D * 3 * 2 + (own_halves<D>() == 2 ? size_t(2 * kWaves) * 16 * 64 * sizeof(float) : 0);
+}
+// A column's running maximum is moved only when a score exceeds it by more than this many powers of two: weights and
+// sums stay below 2^8 times what they would be, and most tiles need no maximum over lanes and no rescaling.
+constexpr float kMaxSlack = 8.f;
+
+template <int D>
+__global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kernel(const OwnArgs a) {
+  constexpr int H = own_halves<D>(), W = kWaves * H, QB = 2;
+  constexpr int NC = D / 32, ND = D / 16, NCH = NC / H, NDH = ND / H;
+  constexpr int KU = 2 * NC / W, VU = ND / W;   // operand blocks of a tile that a wave stages
+  extern __shared__ uint4 own_lds[];
+  bf16x8* const lk = reinterpret_cast<bf16x8*>(own_lds);
+  bf16x8* const lv = lk + 2 * NC * 3 * 64;
+  f32x4* const ex = reinterpret_cast<f32x4*>(lv + ND * 3 * 64);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int rb = wave % kWaves, h = wave / kWaves;
+  const int g = lane >> 4, j = lane & 15;
+
+  // the last (longest) row blocks first
+  const int kvh = int(blockIdx.x) % a.kv_heads, rest = int(blockIdx.x) / a.kv_heads;
+  const int run = rest % a.own, quads = (a.nblocks + kWaves - 1) / kWaves, quad = quads - 1 - rest / a.own;
+  const int blk = quad * kWaves + rb;          // of the launch
+  const int row0 = (a.b0 + blk) * a.rpb;
+  const int cols = blk < a.nblocks ? min(a.rpb, a.n_own - row0) * a.group : 0;
+  const int wg_row0 = (a.b0 + quad * kWaves) * a.rpb;
+  const int wg_last = min(a.n_own, (a.b0 + min(a.nblocks, (quad + 1) * kWaves)) * a.rpb) - 1;
+  // the keys any row of the work-group sees, from a multiple of the tile; this run of them
+  const int k0 = a.window > 0 ? max(0, wg_row0 - a.window + 1) & ~(kTile - 1) : 0;
+  const int kmin = k0 + run * a.run, kmax = min(wg_last + 1, kmin + a.run);
+  const size_t rec0 = (size_t(kvh) * size_t(a.splits1) + size_t(a.splits + run)) * size_t(a.qpad);
+  float* ml = a.ml + (size_t(a.b0 + blk) * a.blk_records + rec0) * 2;
+  if (kmin >= kmax) {   // the whole work-group: no key
+    if (h == 0 && lane < cols) *reinterpret_cast<float2*>(ml + size_t(lane) * 2) = make_float2(-INFINITY, 0.f);
+    return;
+  }
+
+  // a tile's rows, one quarter (or eighth) of the operand blocks a wave; rows past the call's end load its last row
+  // (their scores are masked)
+  const unsigned stride = unsigned(a.kv_heads) * D;
+  auto load_k = [&](int kb, float (&st)[KU][8]) {
+    const float* base = a.k + size_t(kb) * stride + size_t(kvh) * D;
+#pragma unroll
+    for (int u = 0; u < KU; ++u) {
+      const int e = wave + u * W, b = e / NC, c = e % NC;
+      const float* kr = base + (unsigned(min(16 * b + j, a.n_own - 1 - kb)) * stride + unsigned(32 * c + 8 * g));
+      const float4 x = *reinterpret_cast<const float4*>(kr), y = *reinterpret_cast<const float4*>(kr + 4);
+      st[u][0] = x.x, st[u][1] = x.y, st[u][2] = x.z, st[u][3] = x.w;
+      st[u][4] = y.x, st[u][5] = y.y, st[u][6] = y.z, st[u][7] = y.w;
+    }
+  };
+  auto load_v = [&](int kb, float (&st)[VU][8]) {
+    const float* base = a.v + size_t(kb) * stride + size_t(kvh) * D + 16 * wave;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float* vr = base + (unsigned(min(16 * (e >> 2) + 4 * g + (e & 3), a.n_own - 1 - kb)) * stride + unsigned(j));
+#pragma unroll
+      for (int u = 0; u < VU; ++u) st[u][e] = vr[16 * u * W];
+    }
+  };
+  auto put_k = [&](const float (&st)[KU][8]) {
+#pragma unroll
+    for (int u = 0; u < KU; ++u) {
+      bf16x8 t[3];
+      split_exact<true>(st[u], t);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) lk[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
+    }
+  };
+  auto put_v = [&](const float (&st)[VU][8]) {
+#pragma unroll
+    for (int u = 0; u < VU; ++u) {
+      bf16x8 t[3];
+      split_exact<true>(st[u], t);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) lv[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
+    }
+  };
+  static_assert(KU == VU, "one staging array");
+  float st[KU][8];   // the next tile's K until the scores are done, then its V
+  float first_v[VU][8];
+  load_k(kmin, st);
+  load_v(kmin, first_v);
+
+  // the wave's q-cols: operand terms of its dims, and the keys lo .. hi that each column sees
+  bf16x8 q[NCH][QB][3];
+  int lo[QB], hi[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int qc = qb * 16 + j;
+    const bool live = qc < cols;
+    const int i = live ? row0 + qc / a.group : 0;
+    lo[qb] = a.window > 0 ? max(0, i - a.window + 1) : 0;
+    hi[qb] = live ? i : -1;
+    const float* qp = a.q + (size_t(i) * size_t(a.heads) + size_t(kvh * a.group + (live ? qc % a.group : 0))) * D +
+                      32 * h * NCH + 8 * g;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const float4 u = *reinterpret_cast<const float4*>(qp + 32 * c), w = *reinterpret_cast<const float4*>(qp + 32 * c + 4);
+      const float x[8] = {u.x * a.scale2, u.y * a.scale2, u.z * a.scale2, u.w * a.scale2,
+                          w.x * a.scale2, w.y * a.scale2, w.z * a.scale2, w.w * a.scale2};
+      split_exact<true>(x, q[c][qb]);
+    }
+  }
+  put_k(st);
+  put_v(first_v);
+  // wave-uniform: the tiles that hold a key some column sees, and whether all of a tile is seen by every column
+  const int i_first = row0, i_last = cols > 0 ? row0 + (cols - 1) / a.group : -1;
+  const int first_any = a.window > 0 ? max(0, i_first - a.window + 1) : 0;
+  const int last_lo = a.window > 0 ? max(0, i_last - a.window + 1) : 0;
+
+  f32x4 o[QB][NDH];
+  float m[QB], l[QB];   // the column's reference maximum; the lane's share of its sum
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    m[qb] = -INFINITY;
+    l[qb] = 0.f;
+#pragma unroll
+    for (int dd = 0; dd < NDH; ++dd) o[qb][dd] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  __syncthreads();
+  for (int kb = kmin; kb < kmax; kb += kTile) {
+    const bool more = kb + kTile < kmax;
+    const bool any = kb <= i_last && kb + kTile > first_any;   // i_last = -1: a wave without columns
+    f32x4 d[2][QB];
+    if (more) load_k(kb + kTile, st);
+    if (any) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) d[b][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const bf16x8* at = lk + ((b * NC + h * NCH + c) * 3) * 64 + lane;
+          const bf16x8 A[3] = {at[0], at[64], at[128]};
+          mfma_split<QB>(A, q[c], d[b]);
+        }
+      pace_reads<2 * NCH, 6 * QB>();
+      if constexpr (H == 2) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) ex[(wave * 4 + b * 2 + qb) * 64 + lane] = d[b][qb];
+      }
+    }
+    __syncthreads();   // K read by every wave, the V of this tile complete (and the halves' sums)
+    if (more) {
+      put_k(st);
+      load_v(kb + kTile, st);
+    }
+    if (any) {
+      if constexpr (H == 2) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) d[b][qb] += ex[((wave ^ kWaves) * 4 + b * 2 + qb) * 64 + lane];
+      }
+      float s[QB][8];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[qb][e] = d[e >> 2][qb][e & 3];
+      if (kb + kTile - 1 > i_first || kb < last_lo || cols < QB * 16) {   // some key some column does not see
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int key = kb + 16 * (e >> 2) + 4 * g + (e & 3);
+            s[qb][e] = key >= lo[qb] && key <= hi[qb] ? s[qb][e] : -INFINITY;
+          }
+      }
+      bf16x8 p[QB][3];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        float mx = s[qb][0];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s[qb][e]);
+        if (__ballot(mx > m[qb] + kMaxSlack)) {   // some column's maximum moves
+          const float m_new = fmaxf(m[qb], xor32_max(xor16_max(mx)));
+          const float corr = exp2_fast(m[qb] - (m_new == -INFINITY ? 0.f : m_new));
+          m[qb] = m_new;
+          l[qb] *= corr;
+#pragma unroll
+          for (int dd = 0; dd < NDH; ++dd) o[qb][dd] *= corr;
+        }
+        const float m_ref = m[qb] == -INFINITY ? 0.f : m[qb];   // no key of the column yet: weights exp2(-inf) = 0
+        float w[8], ps = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          w[e] = exp2_fast(s[qb][e] - m_ref);
+          ps += w[e];
+        }
+        l[qb] += ps;
+        split_exact<false>(w, p[qb]);
+      }
+#pragma unroll
+      for (int dd = 0; dd < NDH; ++dd) {
+        const bf16x8* at = lv + ((h * NDH + dd) * 3) * 64 + lane;
+        const bf16x8 A[3] = {at[0], at[64], at[128]};
+        f32x4 t[QB];
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) t[qb] = o[qb][dd];
+        mfma_split<QB>(A, p, t);
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) o[qb][dd] = t[qb];
+      }
+      pace_reads<NDH, 6 * QB>();
+    }
+    __syncthreads();   // V (and the halves' sums) read by every wave, the next K complete
+    if (more) put_v(st);
+  }
+
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int qc = qb * 16 + j;
+    const float L = xor32_sum(xor16_sum(l[qb]));
+    if (qc >= cols) continue;
+    float* acc = a.acc + (size_t(a.b0 + blk) * a.blk_records + rec0 + size_t(qc)) * D + 16 * h * NDH;
+    if (h == 0 && g == 0) *reinterpret_cast<float2*>(ml + size_t(qc) * 2) = make_float2(m[qb], L);
+#pragma unroll
+    for (int dd = 0; dd < NDH; ++dd) *reinterpret_cast<f32x4*>(acc + 16 * dd + 4 * g) = o[qb][dd];
+  }
 }
 
 // -------------------------------------------------------------------------------------------------- producer
@@ -1359,9 +1658,18 @@ struct MergeArgs {
   const float* acc;
   const float* ml;
   int heads, group, rpb, kv_heads, splits1, qpad;
+  int own, run, window;    // own-key records, the keys of each (AttnPlan), the call's window
 };
 
-// Chunk c (dims 8c .. 8c + 7 of the row's heads * D outputs) of query row `row`.
+// The records of a row that can hold a key of it: all but the runs of own keys that begin after the row. Its first run
+// begins where its work-group's does (attn_own_kernel: kWaves row blocks).
+__device__ inline int row_records(const MergeArgs& a, int row) {
+  if (a.own == 1) return a.splits1;
+  const int per = kWaves * a.rpb, wg_row0 = row / per * per;
+  const int k0 = a.window > 0 ? max(0, wg_row0 - a.window + 1) & ~(kTile - 1) : 0;
+  return a.splits1 - a.own + min(a.own, (row - k0) / a.run + 1);
+}
+
 // The first record of chunk c (dims 8c .. 8c + 7 of the row's heads * D outputs) of query row `row`.
 template <int D>
 __device__ inline size_t chunk_rec0(const MergeArgs& a, int row, int c) {
@@ -1372,7 +1680,7 @@ __device__ inline size_t chunk_rec0(const MergeArgs& a, int row, int c) {
 
 template <int D, int B>
 __device__ inline void merge_chunk(const MergeArgs& a, int row, int c, float out[8]) {
-  merge8<D, B>(a.acc, a.ml, chunk_rec0<D>(a, row, c), a.qpad, a.splits1, (8 * c) % D, out);
+  merge8<D, B>(a.acc, a.ml, chunk_rec0<D>(a, row, c), a.qpad, row_records(a, row), (8 * c) % D, out);
 }
 
 // One work-group per query row: out[row][heads][D].
@@ -1540,7 +1848,72 @@ __global__ void __launch_bounds__(64 * W) attn_merge_heads_kernel(const MergeArg
 
 // ------------------------------------------------------------------------------------------------------- plan
 
-AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int window) {
+namespace {
+
+// Calls of few rows keep the FP32 kernel, whose waves share nothing and wait for nothing. Whole attention calls, that
+// kernel and the tiled one: 32 rows of 128 dims 10.7 and 13.0 us, 48: 12.5 and 13.2, 64: 14.8 and 13.3; 24 rows of 256
+// dims 17.0 and 17.4, 40: 21.4 and 19.3; 64-dim heads are equal up to 40 rows and the tiled kernel faster above.
+bool own_few_rows(int d, int n_q) { return n_q <= (d == 128 ? 48 : d == 256 ? 32 : 0); }
+
+// The runs of own keys: a work-group of attn_own_kernel (4 row blocks of a KV head) takes one run, and every run of a
+// row is one more record to write and to merge. A run costs its tiles and about kSetup tiles more (the first loads and
+// record); with fewer work-groups than the chip holds at once the longest run is the launch's time, with more the
+// sum over the chip, plus half of a run at the end. A record's write and read back is counted in tiles too. The
+// candidate of the least such time is taken. Whole attention calls without cached keys, runs of 128 keys and the runs
+// taken: 188 rows, 16 / 4 heads of 256: 31.7 and 25.6 us; 256 rows of 128 dims 26 and 23 us; 512 rows, 32 / 8 heads of
+// 128: 42.2 and 37.6 us; 512 rows of 256 dims 46.3 and 48.5 us.
+// With fixed_scratch (the call that allocates nothing, whose array has a fixed size) the count is one run per
+// kOwnChunk keys, as always, so that the same calls fit.
+void plan_own(AttnPlan& p, int n_q, int window, bool fixed_scratch) {
+  const int rows = kWaves * p.rpb;   // of a work-group
+  p.window = window;
+  const long long row_range = window > 0 ? std::min<long long>(n_q, (long long)window + p.rpb - 1) : n_q;
+  const int fixed = int(std::max<long long>(1, (row_range + kOwnChunk - 1) / kOwnChunk));
+  // the keys a work-group's rows see, from a multiple of the tile on
+  const long long range = window > 0 ? std::min<long long>(n_q, (long long)window + rows + kTile - 2) : n_q;
+  const int tiles = int((range + kTile - 1) / kTile);
+  p.own_max = std::max(fixed, std::min(8, tiles));
+  if (own_few_rows(p.d, n_q)) {
+    p.own = 1;
+    p.run = tiles * kTile;
+    return;
+  }
+  if (fixed_scratch) {
+    p.own = p.own_max = fixed;
+    p.run = (tiles + fixed - 1) / fixed * kTile;
+    return;
+  }
+  constexpr double kSetup = 2;
+  const double slots = p.d == 256 ? 256 : 512;   // work-groups the chip holds: one per CU at 256 dims, two below
+  double best = 0;
+  for (int rt = 1;; rt = rt < 4 ? rt + 1 : rt + rt / 2) {   // tiles per run
+    rt = std::min(rt, tiles);
+    const int own = (tiles + rt - 1) / rt;
+    if (own <= p.own_max) {
+      double wgs = 0, work = 0;
+      for (long long r = 0; r < n_q; r += rows) {
+        const long long last = std::min<long long>(n_q, r + rows) - 1;
+        const long long k0 = window > 0 ? std::max<long long>(0, r - window + 1) / kTile * kTile : 0;
+        const double t = double((last - k0) / kTile + 1), n = double((long long)(t + rt - 1) / rt);
+        wgs += n * p.kv_heads;
+        work += (t + n * kSetup) * p.kv_heads;
+      }
+      const double shared = slots > 256 && wgs > 256 ? 1 + 0.3 * (std::min(wgs, slots) - 256) / 256 : 1;
+      const double cost = (wgs <= slots ? rt * shared + kSetup : work / slots * shared + 0.5 * rt) +
+                          wgs * p.d * 6e-5;
+      if (best == 0 || cost < best * 1.01) {   // equal: the fewer records
+        best = cost;
+        p.own = own;
+        p.run = rt * kTile;
+      }
+    }
+    if (rt == tiles) break;
+  }
+}
+
+}  // namespace
+
+AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int window, bool fixed_scratch) {
   XTG_CHECK(c.head_dim == 64 || c.head_dim == 128 || c.head_dim == 256, "attention: head_dim %d (64, 128 or 256)",
             c.head_dim);
   XTG_CHECK(heads % c.kv_heads == 0, "attention: %d heads over %d KV heads", heads, c.kv_heads);
@@ -1587,11 +1960,7 @@ AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int windo
   } else {
     p.splits = 0;
   }
-  // own keys: a column tile's key range is at most the call's rows, or with a window the window and the block's
-  // other rows; the matrix-core own-key kernel takes it in chunks of kOwnChunk keys, a wave each (the producer of a
-  // call of up to kProdRows rows writes the one record itself)
-  const int own_range = window > 0 ? int(std::min<long long>(n_q, (long long)window + p.rpb - 1)) : n_q;
-  p.own = std::max(1, (own_range + kOwnChunk - 1) / kOwnChunk);
+  plan_own(p, n_q, window, fixed_scratch);
   return p;
 }
 
@@ -1717,6 +2086,9 @@ MergeArgs merge_args(const AttnPlan& p, int heads, const float* part) {
   a.kv_heads = p.kv_heads;
   a.splits1 = p.splits + p.own;
   a.qpad = p.qpad;
+  a.own = p.own;
+  a.run = p.run;
+  a.window = p.window;
   return a;
 }
 
@@ -1825,7 +2197,7 @@ std::string launch_attn_scan(const DevKv& c, const AttnPlan& p, int b0, int nblo
 std::string launch_attn_own(const AttnPlan& p, int b0, int nblocks, const float* q, const float* k, const float* v,
                             int n_q, int heads, int window, float scale, float* part, hipStream_t stream) {
   XTG_CHECK(nblocks >= 1 && b0 + nblocks <= p.blocks, "attention: blocks %d .. %d of %d", b0, b0 + nblocks, p.blocks);
-  XTG_CHECK(p.qpad % 16 == 0, "attention: %d padded q-cols", p.qpad);
+  XTG_CHECK(p.qpad % 16 == 0 && b0 % kWaves == 0, "attention: %d padded q-cols, first block %d", p.qpad, b0);
   OwnArgs a{};
   a.q = q;
   a.k = k;
@@ -1844,19 +2216,29 @@ std::string launch_attn_own(const AttnPlan& p, int b0, int nblocks, const float*
   a.splits = p.splits;
   a.splits1 = p.splits + p.own;
   a.qpad = p.qpad;
-  a.tiles = p.qpad / 16;
   a.own = p.own;
+  a.run = p.run;
   a.scale2 = scale * kLog2e;
-  const long long waves = (long long)p.kv_heads * a.tiles * p.own * nblocks;
-  const dim3 grid{unsigned((waves + 3) / 4)}, block{256};
+  if (own_few_rows(p.d, n_q)) {
+    const long long waves = (long long)p.kv_heads * (p.qpad / 16) * nblocks;
+    void (*fn)(const OwnArgs) = p.d == 128 ? attn_own_mfma_kernel<128> : attn_own_mfma_kernel<256>;
+    hipLaunchKernelGGL(fn, dim3(unsigned((waves + 3) / 4)), dim3(256), 0, stream, a);
+    HIP_CHECK(hipGetLastError());
+    return strf("attn_own_mfma_kernel<%d>", p.d);
+  }
+  const long long wgs = (long long)p.kv_heads * p.own * ((nblocks + kWaves - 1) / kWaves);
+  auto launch = [&](void (*fn)(const OwnArgs), int halves, size_t lds) {
+    allow_lds(reinterpret_cast<const void*>(fn), lds);
+    hipLaunchKernelGGL(fn, dim3(unsigned(wgs)), dim3(unsigned(kWaves * halves * 64)), lds, stream, a);
+  };
   if (p.d == 64)
-    hipLaunchKernelGGL(attn_own_mfma_kernel<64>, grid, block, 0, stream, a);
+    launch(attn_own_kernel<64>, own_halves<64>(), own_lds_bytes<64>());
   else if (p.d == 128)
-    hipLaunchKernelGGL(attn_own_mfma_kernel<128>, grid, block, 0, stream, a);
+    launch(attn_own_kernel<128>, own_halves<128>(), own_lds_bytes<128>());
   else
-    hipLaunchKernelGGL(attn_own_mfma_kernel<256>, grid, block, 0, stream, a);
+    launch(attn_own_kernel<256>, own_halves<256>(), own_lds_bytes<256>());
   HIP_CHECK(hipGetLastError());
-  return strf("attn_own_mfma_kernel<%d>", p.d);
+  return strf("attn_own_kernel<%d>", p.d);
 }
 
 std::string launch_attn_merge(const AttnPlan& p, int n_q, int heads, const float* part, float* out,

@@ -40,8 +40,8 @@ std::string launch_kv_store(const DevKv& c, long long pos, int n, const float* k
 
 // How one attention call (n_q query rows at pos0) is cut up. Query rows go in blocks of rpb rows (at most 32
 // (row, head) columns per KV head); each block's key tiles go to `splits` work-groups per KV head, plus `own`
-// partials per (block, KV head) for this call's own keys (one per chunk of kOwnChunk keys of a column tile's key
-// range; chunks with no key leave an empty record, sum 0). Partials: acc [blocks][kv_heads][splits + own][qpad][d]
+// partials per (block, KV head) for this call's own keys (one per run of `run` keys of those that the block's
+// work-group sees; runs with no key leave an empty record, sum 0). Partials: acc [blocks][kv_heads][splits + own][qpad][d]
 // then (max, sum) [blocks][kv_heads][splits + own][qpad][2]; q-col (row r of the block, head g of the group) is
 // r * group + g.
 constexpr int kOwnChunk = 128;
@@ -52,11 +52,14 @@ struct AttnPlan {
   int tile_lo = 0, tiles = 0;  // the 32-slot tiles to scan
   int splits = 0;              // work-groups per KV head over the tiles (0: no cached key is visible)
   int own = 1;                 // own-key records per (block, KV head, q-col), after the splits'
+  int run = 32, window = 0;    // own keys per record, the call's window
+  int own_max = 1;             // what scratch is sized for: grows with the rows only, where `own` goes up and down
   int kv_heads = 1, d = 64;
   size_t records() const { return size_t(blocks) * size_t(kv_heads) * size_t(splits + own) * size_t(qpad); }
-  size_t part_floats() const { return records() * size_t(d + 2); }
+  size_t part_floats() const { return records() / size_t(splits + own) * size_t(splits + own_max) * size_t(d + 2); }
 };
-AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int window);
+// fixed_scratch: for the call whose partials go to the fixed array (one own-key record per kOwnChunk keys).
+AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int window, bool fixed_scratch = false);
 
 // For blocks b0 .. b0 + nblocks - 1 (block b: rows b * rpb .. of the call; device q / k / v as xtg::AttnArgs,
 // engine/include/xtg/kv.h:67-78), one launch each: the own-key partials and the split partials. Then the merge of

@@ -557,7 +557,7 @@ void Backend::check_attention(const DevKv* c, int n_q, long long pos0, const flo
 void Backend::attention_noalloc(const DevKv* c, int n_q, long long pos0, int heads, int window, float scale,
                                 const float* q, const float* k, const float* v, float* out) {
   check_attention(c, n_q, pos0, q, k, v, out);
-  const AttnPlan p = attn_plan(*c, n_q, heads, pos0, window);
+  const AttnPlan p = attn_plan(*c, n_q, heads, pos0, window, true);
   const size_t need = p.part_floats() * sizeof(float);
   XTG_CHECK(need <= kAttnScratchBytes,
             "attention_noalloc: %d rows over %d KV heads (%d key splits) need %zu bytes of partials; the fixed scratch "
