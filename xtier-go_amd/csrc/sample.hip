@@ -28,8 +28,9 @@
 // floor for min_p (max(floor, that) with both): the union is a subset of the row, so the row holds at least as much
 // at or above tau. When in every slice the 64th listed maximum and every thread's second lie below tau, the union
 // holds every weight >= tau, and the candidates are its pairs at or above tau; otherwise they are gathered from
-// the row (at most 4096, sorted in LDS), or, past that, the whole row is sorted by a stable LSD radix sort in scratch
-// memory (8 passes of 4 bits): slower, the same result. Sorts in LDS are merges of sorted runs of 64 (the slices'
+// the row (at most 4096, sorted in LDS), or, past that, the sums are found by counting (wide_find), or, for a top_k past
+// that and the cases wide_find leaves, the whole row is sorted by a stable LSD radix sort in scratch memory (8 passes of
+// 4 bits): slower, the same result. Sorts in LDS are merges of sorted runs of 64 (the slices'
 // lists as they come; gathered pairs sorted by the waves in registers first), one barrier per doubling of the run
 // instead of one per stage of a bitonic network over the whole set (78 for 4096 pairs). Greedy rows take the
 // slices' first maxima (argmax_pick_kernel).
@@ -431,11 +432,141 @@ __device__ inline float union_select(const float* __restrict__ uw, int U, bool m
 }
 }  // namespace
 
+constexpr int kCand = 4096;   // candidates sorted in LDS
+
+namespace {
+// Running sums in candidate order without sorting the row, for filters that keep more candidates than fit in LDS, or
+// whose threshold the slices' lists do not give. Weights (in [0, 1]) are counted by the bits of their value, 256
+// buckets a level, most likely first: at the top 8 of an octave over 32 octaves (bits >> 20), and where a bucket holds
+// more than kCand, 256 of it by its next 8 bits. All weights of a bucket have one exponent, so its mass is an integer
+// sum of 24-bit mantissas: exact, in any order, and with n < 2^20 it fits 44 bits with the count above it. The bucket
+// where the running sum crosses is gathered, sorted in LDS and walked from the mass above it.
+// One work-group reads the row once per level and once per gather (131072 weights: about 7 us each); 32 copies of each
+// counter, one per bank pair, keep the lanes of a wave off each other's. Measured, whole calls, stable sort of the
+// whole row before and now: 131072 weights at top_p 0.95 with 11000 kept, 2808 and 94 us; 32000 weights 683 and 52 us;
+// 8 rows of 131072 2870 and 100 us.
+constexpr int kWideRow = 1 << 20;   // rows below this length
+struct WideLevel {
+  double pre[257];     // mass above each bucket, and above the end
+  uint32_t cnt[256];   // weights in each
+};
+
+// Counts the weights w[0, n) >= floor_w whose bits >> (sh + 8) equal `prefix` (all, at the top level: sh = 20) into L,
+// from `base` up. The top level's last bucket takes everything below 2^-31.75: its mass counts as nothing. h: LDS,
+// 256 * 32 counters. Every thread of the work-group.
+__device__ inline void wide_count(const float* w, int n, float floor_w, int sh, uint32_t prefix, double base, WideLevel& L,
+                                  unsigned long long* h) {
+  const int t = int(threadIdx.x);
+  const bool top = sh == 20;
+  __syncthreads();   // h and L free
+  for (int q = t; q < 256 * 32; q += kSampleThreads) h[q] = 0;
+  __syncthreads();
+  for (int i0 = t; i0 < n; i0 += 8 * kSampleThreads) {
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = i0 + u * kSampleThreads < n ? w[i0 + u * kSampleThreads] : -1.f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint32_t bits = __float_as_uint(x[u]);
+      if (x[u] >= floor_w && x[u] >= 0.f && (top || bits >> (sh + 8) == prefix)) {
+        const int b = top ? min(255, 0x3f8 - int(bits >> 20)) : 255 - int(bits >> sh & 255u);
+        atomicAdd(&h[b * 32 + (t & 31)], 1ull << 44 | ((bits & 0x7fffffu) | 0x800000u));
+      }
+    }
+  }
+  __syncthreads();
+  if (t < 256) {
+    unsigned long long c = 0;
+    for (int q = 0; q < 32; ++q) c += h[t * 32 + ((q + t) & 31)];
+    const int e = top ? (0x3f8 - t) >> 3 : int(prefix << (sh + 8) >> 23);   // the bucket's biased exponent
+    const double unit = __longlong_as_double((long long)(e - 150 + 1023) << 52);
+    L.cnt[t] = uint32_t(c >> 44);
+    L.pre[t + 1] = top && t == 255 ? 0.0 : double(c & ((1ull << 44) - 1)) * unit;
+  }
+  __syncthreads();
+  if (t == 0) {
+    double c = base;
+    L.pre[0] = c;
+    for (int b = 1; b <= 256; b += 16) {
+      double v[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) v[q] = L.pre[b + q];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) L.pre[b + q] = c += v[q];
+    }
+  }
+  __syncthreads();
+}
+
+// The first candidate (of those >= floor_w, in candidate order) at which the running sum is > r (strict) or >= r, or
+// the last one when none: its pair key, and in *at the running sum there; kPadKey when the sum crosses among weights
+// below 2^-31.75 or more than kCand weights agree in all but 4 bits. top: the row's top level, counted; sub: a level of
+// scratch; ck: LDS for kCand keys; h: LDS for 256 * 32 counters (the sort's scratch, too). Every thread.
+__device__ inline unsigned long long wide_find(const float* w, int n, float floor_w, double r, bool strict,
+                                               const WideLevel& top, WideLevel& sub, unsigned long long* ck,
+                                               unsigned long long* h, double* red, int* sel, int* count, double* at) {
+  const int t = int(threadIdx.x), lane = t & 63;
+  const WideLevel* L = &top;
+  int sh = 20;
+  uint32_t pick = 0;   // the chosen bucket: bits >> sh
+  double base = 0.0;
+  int c = 0;
+  for (;;) {
+    __syncthreads();
+    if (t == 0) *sel = INT_MAX, *count = -1;
+    __syncthreads();
+    const bool rest = sh == 20;   // the top level's last bucket
+    if (t < 256 && L->cnt[t]) {
+      if (!(rest && t == 255) && (strict ? L->pre[t + 1] > r : L->pre[t + 1] >= r)) atomicMin(sel, t);
+      atomicMax(count, t);
+    }
+    __syncthreads();
+    int b = *sel;
+    if (b == INT_MAX) b = *count;   // no crossing: the last bucket with any
+    if (b < 0 || (rest && b == 255)) return kPadKey;
+    base = L->pre[b];
+    c = int(L->cnt[b]);
+    pick = rest ? uint32_t(0x3f8 - b) : (pick << 8 | uint32_t(255 - b));
+    if (c <= kCand) break;
+    if (sh == 4) return kPadKey;
+    sh -= 8;
+    wide_count(w, n, floor_w, sh, pick, base, sub, h);
+    L = &sub;
+  }
+  __syncthreads();
+  if (t == 0) *count = 0;
+  __syncthreads();
+  for (int i0 = t; i0 - t < n; i0 += 8 * kSampleThreads) {   // the same rounds in every thread
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = i0 + u * kSampleThreads < n ? w[i0 + u * kSampleThreads] : -1.f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const bool in = x[u] >= floor_w && __float_as_uint(x[u]) >> sh == pick;
+      const unsigned long long m = __ballot(in);
+      if (m) {
+        int at0 = 0;
+        if (lane == 0) at0 = atomicAdd(count, __popcll(m));
+        at0 = __shfl(at0, 0);
+        if (in) ck[at0 + __popcll(m & ((1ull << lane) - 1))] = pair_key(x[u], i0 + u * kSampleThreads);
+      }
+    }
+  }
+  int n2 = 1;
+  while (n2 < c) n2 <<= 1;
+  for (int q = c + t; q < n2; q += kSampleThreads) ck[q] = kPadKey;
+  sort_pairs<kSampleThreads>(ck, h, n2);
+  const int i = first_crossing([&](int j) { return key_w(ck[j]); }, c, r, strict, red, sel, at, base);
+  const unsigned long long key = ck[i < c ? i : c - 1];
+  __syncthreads();   // ck free
+  return key;
+}
+}  // namespace
+
 // Per-row scratch (floats / ints / doubles laid out by SampleScratch): the weights, and per slice of kSlice logits
 // its max, argmax, weight sum, count and mass at or above the min_p floor, its 64 largest thread maxima in
 // candidate order (-1 weights past the slice's threads) and the largest second-most-likely weight of a thread.
 constexpr int kSlice = 2048, kSliceThreads = 256, kSliceTop = 64;
-constexpr int kCand = 4096;   // candidates sorted in LDS
 
 struct SampleArgs {
   const float* logits;   // [rows][n]
@@ -625,6 +756,8 @@ __global__ void __launch_bounds__(kSampleThreads) sample_pick_kernel(const Sampl
   __shared__ unsigned long long ck[kCand];   // candidates as pair keys
   unsigned long long* tk = reinterpret_cast<unsigned long long*>(hist);
   __shared__ unsigned long long selh[256];
+  static_assert(256 * 32 * 2 <= 16 * kSampleThreads, "counters in hist");
+  __shared__ WideLevel wide[2];
   __shared__ int sel, ccount, slices_ok, nread;
   __shared__ unsigned long long above_s;
   __shared__ double base_s;
@@ -868,6 +1001,26 @@ __global__ void __launch_bounds__(kSampleThreads) sample_pick_kernel(const Sampl
       sort_pairs<kSampleThreads>(ck, tk, n2);
       L = nc;
     } else {
+      // a sum over more: by counting (a NaN or infinite total has a NaN among the weights: the sort takes it)
+      if (!topk && n < kWideRow && total < INFINITY) {
+        unsigned long long* h = reinterpret_cast<unsigned long long*>(hist);
+        const float fl = a.min_p > 0.f ? floor_w : 0.f;
+        double sum = a.min_p > 0.f ? t_floor : total, at = 0.0;
+        unsigned long long last = kPadKey - 1;   // the last kept candidate
+        wide_count(w, n, fl, 20, 0, 0.0, wide[0], h);
+        if (a.top_p < 1.f) {
+          last = wide_find(w, n, fl, sum * double(a.top_p), false, wide[0], wide[1], ck, h, red, &sel, &ccount, &at);
+          sum = at;
+        }
+        const unsigned long long key =
+            last == kPadKey ? kPadKey
+                            : wide_find(w, n, fl, a.u[row] * sum, true, wide[0], wide[1], ck, h, red, &sel, &ccount, &at);
+        if (key != kPadKey) {
+          if (t == 0) a.out[row] = key_id(key < last ? key : last);
+          return;
+        }
+        __syncthreads();
+      }
       // the whole row, stably sorted by (~bits(w), index), 4 bits a pass, contiguous chunks per thread
       uint32_t* k0 = a.keys + size_t(row) * 2 * size_t(n);
       uint32_t* k1 = k0 + n;
