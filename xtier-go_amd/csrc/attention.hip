@@ -1142,14 +1142,14 @@ __device__ inline void mfma_split(const bf16x8 (&A)[3], const bf16x8 (&B)[QB][3]
     for (int qb = 0; qb < QB; ++qb) d[qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[ta[n]], B[qb][tb[n]], d[qb], 0, 0, 0);
 }
 
-// The order of N groups of 3 operand reads and M matrix ops: each group's reads go out before the matrix ops of the
+// The order of N groups of R operand reads and M matrix ops: each group's reads go out before the matrix ops of the
 // group before (the compiler by itself waits for a group's reads right before its first matrix op).
-template <int N, int M>
+template <int N, int M, int R>
 __device__ __forceinline__ void pace_reads() {
-  __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // LDS reads
+  __builtin_amdgcn_sched_group_barrier(0x100, R, 0);   // LDS reads
 #pragma unroll
   for (int n = 1; n < N; ++n) {
-    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, R, 0);
     __builtin_amdgcn_sched_group_barrier(0x8, M, 0);   // matrix ops
   }
   __builtin_amdgcn_sched_group_barrier(0x8, M, 0);
@@ -1302,7 +1302,7 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
           const bf16x8 A[3] = {at[0], at[64], at[128]};
           mfma_split<QB>(A, q[c], d[b]);
         }
-      pace_reads<2 * NCH, 6 * QB>();
+      pace_reads<2 * NCH, 6 * QB, 3>();
       if constexpr (H == 2) {
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -1371,7 +1371,7 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) o[qb][dd] = t[qb];
       }
-      pace_reads<NDH, 6 * QB>();
+      pace_reads<NDH, 6 * QB, 3>();
     }
     __syncthreads();   // V (and the halves' sums) read by every wave, the next K complete
     if (more) put_v(st);
@@ -1386,6 +1386,278 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
     if (h == 0 && g == 0) *reinterpret_cast<float2*>(ml + size_t(qc) * 2) = make_float2(m[qb], L);
 #pragma unroll
     for (int dd = 0; dd < NDH; ++dd) *reinterpret_cast<f32x4*>(acc + 16 * dd + 4 * g) = o[qb][dd];
+  }
+}
+
+// ----------------------------------------------------------------------------------------------- scan, many rows
+
+// The scan of calls of many rows (AttnPlan::quads): as attn_own_kernel, 4 consecutive row blocks of a KV head share
+// every tile through LDS, double-buffered, instead of each reading it from the caches into its own registers (16 KB a
+// tile and wave at 128 dims and BF16: 80 % of what a CU's vector cache delivers while the matrix ops run). 8 waves:
+// at 64 and 128 dims two per row block, one for the even and one for the odd tiles of the split (KH), merged in LDS at
+// the end; at 256 dims two per row block with half of the dims each (H, as own_halves). BF16 tiles go into LDS by
+// direct loads; FP8 codes are converted to BF16 once on the way. Terms and matrix ops are the scan's: q in three terms,
+// the weights in two. On the vector ALUs, beside which the matrix ops run: no mask where a tile is seen whole, nothing
+// taken over the column's lanes but a maximum that moves, and the sums once at the end.
+// Measured, 512 rows, whole calls: 3000 BF16 keys of 32 / 8 heads of 128 121 -> 101 us (the kernel alone 98 -> 67 us,
+// 63 GFLOP of matrix ops issued: 0.95 PFLOP/s), of 16 / 4 heads of 256 141 -> 126 us; 8000 keys of 128 dims 248 -> 178
+// us; a full ring of 1040 FP8 slots of 256 dims 85 -> 66 us. Bound by the vector ALUs and the matrix ops about evenly.
+template <int D>
+constexpr int rows_key_halves() { return own_halves<D>() == 2 ? 1 : 2; }
+template <int D>
+constexpr int rows_step_blocks() { return rows_key_halves<D>() * (2 * (D / 32) + D / 16); }   // of 64 x 16 bytes
+// Blocks of the two buffers, or of the odd tiles' states that pass through them at the end.
+template <int D>
+constexpr int rows_buf_blocks() {
+  return rows_key_halves<D>() == 2 ? std::max(2 * rows_step_blocks<D>(), kWaves * (2 * (D / 16) + 1)) : 2 * rows_step_blocks<D>();
+}
+template <int D>
+constexpr size_t rows_lds_bytes() {
+  return size_t(rows_buf_blocks<D>()) * 1024 + (own_halves<D>() == 2 ? size_t(2 * kWaves) * 16 * 64 * sizeof(float) : 0) +
+         2 * 3 * 64 * sizeof(float);
+}
+
+template <int D, bool F8>
+__global__ void __launch_bounds__(2 * kWaves * 64, 2) attn_scan_rows_kernel(const ScanArgs a, int nblocks, int kv_heads) {
+  constexpr int H = own_halves<D>(), KH = rows_key_halves<D>(), W = 2 * kWaves, QB = 2;
+  constexpr int NC = D / 32, ND = D / 16, NCH = NC / H, NDH = ND / H, TB = 2 * NC + ND;   // blocks of a tile
+  constexpr int SB = rows_step_blocks<D>(), LU = (F8 ? SB / 2 : SB) / W;   // blocks of a step; loads of a wave
+  extern __shared__ uint4 rows_lds[];
+  bf16x8* const bufs = reinterpret_cast<bf16x8*>(rows_lds);
+  f32x4* const ex = reinterpret_cast<f32x4*>(bufs + rows_buf_blocks<D>() * 64);
+  int* const spos = reinterpret_cast<int*>(ex + (H == 2 ? W * 4 * 64 : 0));   // [2][64]
+  float* const sks = reinterpret_cast<float*>(spos + 128);
+  float* const svs = sks + 128;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int rb = wave % kWaves, half = wave / kWaves, h = H == 2 ? half : 0, kh = H == 2 ? 0 : half;
+  const int g = lane >> 4, j = lane & 15;
+  const int kvh = int(blockIdx.x) % kv_heads, rest = int(blockIdx.x) / kv_heads;
+  const int split = rest % a.splits, quad = rest / a.splits;
+  const int blk = quad * kWaves + rb, row0 = (a.b0 + blk) * a.rpb;
+  const int cols = blk < nblocks ? min(a.rpb, a.n_q - row0) * a.group : 0;
+  const int t_begin = a.tile_lo + int((long long)a.tiles * split / a.splits);
+  const int t_end = a.tile_lo + int((long long)a.tiles * (split + 1) / a.splits);
+  const size_t head_u4 = size_t(a.slots_pad) * size_t(D) / (F8 ? 16 : 8);
+  const uint4* const kbase = a.ck + size_t(kvh) * head_u4;
+  const uint4* const vbase = a.cv + size_t(kvh) * head_u4;
+  const float* const ksb = F8 ? a.kscale + size_t(kvh) * size_t(a.slots_pad) : nullptr;
+  const float* const vsb = F8 ? a.vscale + size_t(kvh) * size_t(a.slots_pad) : nullptr;
+
+  // a step's tiles t0 .. t0 + KH - 1 (past the split's end: its last tile again, not used)
+  uint4 codes[F8 ? LU : 1];
+  int side = 0;   // wave 0: slot positions, waves 1 and 2: scales (as bits)
+  auto load = [&](int t0, int p) {
+    constexpr int LB = F8 ? TB / 2 : TB;   // 16-byte blocks of a tile in memory
+#pragma unroll
+    for (int i = 0; i < LU; ++i) {
+      const int e = wave + i * W, tile = min(t0 + e / LB, t_end - 1), r = e % LB;
+      constexpr int KB = F8 ? NC : 2 * NC;   // of them K's
+      const uint4* src = r < KB ? kbase + (size_t(tile) * KB + size_t(r)) * 64 : vbase + (size_t(tile) * (LB - KB) + size_t(r - KB)) * 64;
+      if constexpr (F8)
+        codes[i] = src[lane];
+      else
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + lane),
+                                         (__attribute__((address_space(3))) void*)(bufs + (p * SB + e) * 64), 16, 0, 0);
+    }
+    const int slot = min(t0 + lane / kTile, t_end - 1) * kTile + lane % kTile;
+    if (wave == 0) side = a.slot_pos[slot];
+    if constexpr (F8) {
+      if (wave == 1) side = __float_as_int(ksb[slot]);
+      if (wave == 2) side = __float_as_int(vsb[slot]);
+    }
+  };
+  auto put = [&](int p) {
+    if constexpr (F8) {
+      constexpr int LB = TB / 2;
+#pragma unroll
+      for (int i = 0; i < LU; ++i) {   // block r of a tile holds the operand blocks 2 r and 2 r + 1
+        const int e = wave + i * W;
+        bf16x8* at = bufs + (p * SB + e / LB * TB + e % LB * 2) * 64 + lane;
+        at[0] = fp8x8_to_bf16(codes[i].x, codes[i].y);
+        at[64] = fp8x8_to_bf16(codes[i].z, codes[i].w);
+      }
+    }
+    if (wave < (F8 ? 3 : 1)) spos[wave * 128 + p * 64 + lane] = side;
+  };
+  load(t_begin, 0);
+
+  bf16x8 q[NCH][QB][3];
+  int lo[QB];
+  const int last_row = a.pos0 + row0 + (cols > 0 ? (cols - 1) / a.group : 0);
+  const int lo_all = a.window > 0 ? max(0, last_row - a.window + 1) : 0;   // every column sees positions from here
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int qc = qb * 16 + j;
+    const bool live = qc < cols;
+    const int i = live ? row0 + qc / a.group : 0;
+    lo[qb] = !live ? INT_MAX : (a.window > 0 ? max(0, a.pos0 + i - a.window + 1) : 0);
+    const float* qp = a.q + (size_t(i) * size_t(a.heads) + size_t(kvh * a.group + (live ? qc % a.group : 0))) * D +
+                      32 * h * NCH + 8 * g;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const float4 u = *reinterpret_cast<const float4*>(qp + 32 * c), w = *reinterpret_cast<const float4*>(qp + 32 * c + 4);
+      const float x[8] = {u.x * a.scale2, u.y * a.scale2, u.z * a.scale2, u.w * a.scale2,
+                          w.x * a.scale2, w.y * a.scale2, w.z * a.scale2, w.w * a.scale2};
+      split_exact<true>(x, q[c][qb]);
+    }
+  }
+  f32x4 o[QB][NDH];
+  float m[QB], l[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    m[qb] = -INFINITY;
+    l[qb] = 0.f;
+#pragma unroll
+    for (int dd = 0; dd < NDH; ++dd) o[qb][dd] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  put(0);
+
+  for (int t0 = t_begin, p = 0; t0 < t_end; t0 += KH, p ^= 1) {
+    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): this wave's share of the step is in LDS
+    __syncthreads();                      // and everyone's; the other buffer is read
+    const bool more = t0 + KH < t_end, any = cols > 0 && t0 + kh < t_end;
+    const int key0 = p * 64 + kh * kTile + 4 * g;   // the lane's keys: key0 + 16 b + 0 .. 3
+    // read before the next step's loads go out (behind loads into LDS the compiler waits for them)
+    const int4 p0 = *reinterpret_cast<const int4*>(spos + key0), p1 = *reinterpret_cast<const int4*>(spos + key0 + 16);
+    if (more) load(t0 + KH, p ^ 1);
+    const bf16x8* const tile = bufs + (p * SB + kh * TB) * 64 + lane;
+    f32x4 d[2][QB];
+    if (any) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) d[b][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const bf16x8 A = tile[(b * NC + h * NCH + c) * 64];
+#pragma unroll
+          for (int term = 2; term >= 0; --term)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb)
+              d[b][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, q[c][qb][term], d[b][qb], 0, 0, 0);
+        }
+      pace_reads<NCH, 2 * 3 * QB, 2>();
+      if constexpr (H == 2) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) ex[(wave * 4 + b * 2 + qb) * 64 + lane] = d[b][qb];
+      }
+    }
+    if constexpr (H == 2) __syncthreads();
+    if (any) {
+      if constexpr (H == 2) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) d[b][qb] += ex[((wave ^ kWaves) * 4 + b * 2 + qb) * 64 + lane];
+      }
+      const int kpos[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+      float s[QB][8];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[qb][e] = d[e >> 2][qb][e & 3];
+      if constexpr (F8) {
+        const float4 k0 = *reinterpret_cast<const float4*>(sks + key0), k1 = *reinterpret_cast<const float4*>(sks + key0 + 16);
+        const float ks[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) s[qb][e] *= ks[e];
+      }
+      const int least = min(min(min(kpos[0], kpos[1]), min(kpos[2], kpos[3])), min(min(kpos[4], kpos[5]), min(kpos[6], kpos[7])));
+      const int most = max(max(max(kpos[0], kpos[1]), max(kpos[2], kpos[3])), max(max(kpos[4], kpos[5]), max(kpos[6], kpos[7])));
+      if (cols < QB * 16 || __ballot(least < lo_all || most >= a.pos0)) {   // some key some column does not see
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) s[qb][e] = kpos[e] >= lo[qb] && kpos[e] < a.pos0 ? s[qb][e] : -INFINITY;
+      }
+      bf16x8 phi[QB], plo[QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        float mx = s[qb][0];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s[qb][e]);
+        if (__ballot(mx > m[qb])) {   // some column's maximum moves (the weight of the largest is then 1, exact in one term)
+          const float m_new = fmaxf(m[qb], xor32_max(xor16_max(mx)));
+          const float corr = exp2_fast(m[qb] - (m_new == -INFINITY ? 0.f : m_new));
+          m[qb] = m_new;
+          l[qb] *= corr;
+#pragma unroll
+          for (int dd = 0; dd < NDH; ++dd) o[qb][dd] *= corr;
+        }
+        const float m_ref = m[qb] == -INFINITY ? 0.f : m[qb];   // nothing visible yet: weights exp2(-inf) = 0
+        float w[8], ps = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          w[e] = exp2_fast(s[qb][e] - m_ref);
+          ps += w[e];
+        }
+        l[qb] += ps;
+        if constexpr (F8) {
+          const float4 v0 = *reinterpret_cast<const float4*>(svs + key0), v1 = *reinterpret_cast<const float4*>(svs + key0 + 16);
+          w[0] *= v0.x, w[1] *= v0.y, w[2] *= v0.z, w[3] *= v0.w, w[4] *= v1.x, w[5] *= v1.y, w[6] *= v1.z, w[7] *= v1.w;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const __bf16 t = to_bf16(w[e]);
+          phi[qb][e] = t;
+          plo[qb][e] = to_bf16(w[e] - of_bf16(t));
+        }
+      }
+#pragma unroll
+      for (int dd = 0; dd < NDH; ++dd) {
+        const bf16x8 A = tile[(2 * NC + h * NDH + dd) * 64];
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) o[qb][dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, plo[qb], o[qb][dd], 0, 0, 0);
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) o[qb][dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, phi[qb], o[qb][dd], 0, 0, 0);
+      }
+      pace_reads<NDH / 2, 2 * 2 * QB, 2>();
+    }
+    if (more) put(p ^ 1);
+  }
+
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) l[qb] = xor32_sum(xor16_sum(l[qb]));
+  if constexpr (KH == 2) {   // the odd tiles' states to the even tiles' waves, through the buffers
+    constexpr int per = QB * NDH + 1;   // f32x4 a lane: outputs, then (m, l) of the two column blocks
+    static_assert(kWaves * per <= rows_buf_blocks<D>(), "states in the buffers");
+    f32x4* const hand = reinterpret_cast<f32x4*>(bufs) + rb * per * 64 + lane;
+    __syncthreads();   // the last step read
+    if (half == 1) {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int dd = 0; dd < NDH; ++dd) hand[(qb * NDH + dd) * 64] = o[qb][dd];
+      hand[QB * NDH * 64] = f32x4{m[0], l[0], m[1], l[1]};
+    }
+    __syncthreads();
+    if (half == 1) return;
+    const f32x4 other = hand[QB * NDH * 64];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const float m1 = other[2 * qb], M = fmaxf(m[qb], m1), ref = M == -INFINITY ? 0.f : M;
+      const float f0 = exp2_fast(m[qb] - ref), f1 = exp2_fast(m1 - ref);
+      m[qb] = M;
+      l[qb] = l[qb] * f0 + other[2 * qb + 1] * f1;
+#pragma unroll
+      for (int dd = 0; dd < NDH; ++dd) o[qb][dd] = o[qb][dd] * f0 + hand[(qb * NDH + dd) * 64] * f1;
+    }
+  }
+  const size_t rec0 = size_t(a.b0 + blk) * a.blk_records + (size_t(kvh) * size_t(a.splits1) + size_t(split)) * size_t(a.qpad);
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int qc = qb * 16 + j;
+    if (qc >= cols) continue;
+    if (h == 0 && g == 0) *reinterpret_cast<float2*>(a.ml + (rec0 + size_t(qc)) * 2) = make_float2(m[qb], l[qb]);
+    float* acc = a.acc + (rec0 + size_t(qc)) * D + 16 * h * NDH + 4 * g;
+#pragma unroll
+    for (int dd = 0; dd < NDH; ++dd) *reinterpret_cast<f32x4*>(acc + 16 * dd) = o[qb][dd];
   }
 }
 
@@ -1658,16 +1930,21 @@ struct MergeArgs {
   const float* acc;
   const float* ml;
   int heads, group, rpb, kv_heads, splits1, qpad;
-  int own, run, window;    // own-key records, the keys of each (AttnPlan), the call's window
+};
+
+// What the merges of many-row calls know beside it (apart, so that the one-block merges' arguments stay in one
+// 64-byte line): own-key records, the keys of each (AttnPlan), the call's window.
+struct OwnRuns {
+  int own, run, window;
 };
 
 // The records of a row that can hold a key of it: all but the runs of own keys that begin after the row. Its first run
 // begins where its work-group's does (attn_own_kernel: kWaves row blocks).
-__device__ inline int row_records(const MergeArgs& a, int row) {
-  if (a.own == 1) return a.splits1;
+__device__ inline int row_records(const MergeArgs& a, const OwnRuns& r, int row) {
+  if (r.own == 1) return a.splits1;
   const int per = kWaves * a.rpb, wg_row0 = row / per * per;
-  const int k0 = a.window > 0 ? max(0, wg_row0 - a.window + 1) & ~(kTile - 1) : 0;
-  return a.splits1 - a.own + min(a.own, (row - k0) / a.run + 1);
+  const int k0 = r.window > 0 ? max(0, wg_row0 - r.window + 1) & ~(kTile - 1) : 0;
+  return a.splits1 - r.own + min(r.own, (row - k0) / r.run + 1);
 }
 
 // The first record of chunk c (dims 8c .. 8c + 7 of the row's heads * D outputs) of query row `row`.
@@ -1679,17 +1956,17 @@ __device__ inline size_t chunk_rec0(const MergeArgs& a, int row, int c) {
 }
 
 template <int D, int B>
-__device__ inline void merge_chunk(const MergeArgs& a, int row, int c, float out[8]) {
-  merge8<D, B>(a.acc, a.ml, chunk_rec0<D>(a, row, c), a.qpad, row_records(a, row), (8 * c) % D, out);
+__device__ inline void merge_chunk(const MergeArgs& a, const OwnRuns& r, int row, int c, float out[8]) {
+  merge8<D, B>(a.acc, a.ml, chunk_rec0<D>(a, row, c), a.qpad, row_records(a, r, row), (8 * c) % D, out);
 }
 
 // One work-group per query row: out[row][heads][D].
 template <int D>
-__global__ void __launch_bounds__(kMergeThreads) attn_merge_kernel(const MergeArgs a, float* __restrict__ out) {
+__global__ void __launch_bounds__(kMergeThreads) attn_merge_kernel(const MergeArgs a, const OwnRuns r, float* __restrict__ out) {
   const int row = blockIdx.x, Q = a.heads * D;
   for (int c = threadIdx.x; c < Q / 8; c += kMergeThreads) {
     float o[8];
-    merge_chunk<D, 12>(a, row, c, o);
+    merge_chunk<D, 12>(a, r, row, c, o);
     float* p = out + size_t(row) * Q + 8 * c;
     *reinterpret_cast<float4*>(p) = make_float4(o[0], o[1], o[2], o[3]);
     *reinterpret_cast<float4*>(p + 4) = make_float4(o[4], o[5], o[6], o[7]);
@@ -1702,7 +1979,7 @@ template <int D, int U>
 __global__ void __launch_bounds__(kMergeThreads) attn_gate_kernel(const MergeArgs a, const float* __restrict__ g,
                                                                    const float* __restrict__ gs, int vec,
                                                                    float* __restrict__ out, f16x8* __restrict__ xop,
-                                                                   float* __restrict__ xinv, size_t ostride) {
+                                                                   float* __restrict__ xinv, size_t ostride, const OwnRuns r) {
   __shared__ float red[2 * kMergeThreads / 64];
   const int row = blockIdx.x, Q = a.heads * D;
   float gv[U][8], sv[U][8], t[U][8];
@@ -1712,7 +1989,7 @@ __global__ void __launch_bounds__(kMergeThreads) attn_gate_kernel(const MergeArg
   for (int u = 0; u < U; ++u) {
     const int c = int(threadIdx.x) + u * kMergeThreads;
     if (8 * c < Q) {
-      merge_chunk<D, (U == 1 ? 12 : 16 / (2 * U))>(a, row, c, t[u]);
+      merge_chunk<D, (U == 1 ? 12 : 16 / (2 * U))>(a, r, row, c, t[u]);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) t[u][e] = 0.f;
@@ -1929,10 +2206,14 @@ AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int windo
   p.rpb = std::max(1, 32 / group);
   p.blocks = (n_q + p.rpb - 1) / p.rpb;
   p.qpad = (std::min(n_q, p.rpb) * group + 15) / 16 * 16;
-  if (c.ring) {   // any slot may hold a visible position: scan the whole ring
+  // a ring's tiles: any slot may hold a visible position once it has wrapped. Before that, as in a cache by position,
+  // positions lo(pos0) .. pos0 - 1 live in slots of the same number: many-row calls scan only those (a prompt's first
+  // chunk none: 512 rows over an empty ring of 1040 FP8 slots, 37 us of a scan that saw nothing).
+  const int ring_tiles = c.slots_pad / kTile;
+  if (c.ring && (pos0 > c.slots || n_q <= kProdRows)) {
     p.tile_lo = 0;
-    p.tiles = c.slots_pad / kTile;
-  } else {        // positions lo(pos0) .. pos0 - 1 live in slots of the same number
+    p.tiles = ring_tiles;
+  } else {
     long long lo = window > 0 ? std::max<long long>(0, pos0 - window + 1) : 0;   // row 0 sees the earliest key
     lo = std::max<long long>(0, std::min<long long>(lo, pos0));
     const long long hi = std::min<long long>(pos0, c.slots);
@@ -1950,16 +2231,29 @@ AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int windo
   // 8 %, and 512 work-groups take 1.5 % off the one-token step at 32K (1.099 -> 1.082 ms, with the gate's merge on
   // more waves; 0.2 % at 8K; 768 and 1024: 1.109 and 1.105 ms), while at 8 rows they cost 4 %.
   // (XTG_ATTN_SPLITS=n fixes the count, for experiments)
-  if (p.tiles > 0) {
+  auto splits_of = [&](int tiles) {
     const int wgs = c.fp8 && !c.ring && n_q == 1 ? 512 : 192;
     const int want = std::max(1, wgs / (c.kv_heads * p.blocks));   // about wgs work-groups over all blocks
     const int mt = c.ring ? 1 : 2;
-    p.splits = std::max(1, std::min(want, (p.tiles + mt * kWaves - 1) / (mt * kWaves)));
-    if (const char* env = std::getenv("XTG_ATTN_SPLITS")) p.splits = std::max(1, std::atoi(env));
-    p.splits = std::min(p.splits, p.tiles);
+    int n = std::max(1, std::min(want, (tiles + mt * kWaves - 1) / (mt * kWaves)));
+    if (const char* env = std::getenv("XTG_ATTN_SPLITS")) n = std::max(1, std::atoi(env));
+    return std::min(n, tiles);
+  };
+  if (p.tiles > 0) {
+    p.splits = splits_of(p.tiles);
+    // calls of many rows share their tiles (attn_scan_rows_kernel), a work-group per CU with at least 4 tiles each.
+    // Whole calls, each on its own tiles and shared: 64 rows over 1500 keys 29.9 and 36 us (128 dims), 47.6 and 55 us
+    // (256); 96 rows 36.6 and 37.9; 128 rows 48 and 43 us, 77 and 54 us; 128 dims and few tiles, 256 rows over 300
+    // keys, 40 and 43 us, where 256 dims take 71 and 58 us. (The fixed array's calls keep the plan that fits it.)
+    const int quads = c.kv_heads * ((p.blocks + kWaves - 1) / kWaves);
+    p.quads = !fixed_scratch && n_q >= 128 && (c.head_dim != 128 || p.tiles >= 32);
+    if (p.quads && !std::getenv("XTG_ATTN_SPLITS")) {
+      p.splits = std::max(1, std::min(256 / quads, p.tiles / 4));
+    }
   } else {
     p.splits = 0;
   }
+  p.splits_max = c.ring ? std::max(p.splits, splits_of(ring_tiles)) : p.splits;
   plan_own(p, n_q, window, fixed_scratch);
   return p;
 }
@@ -2086,11 +2380,10 @@ MergeArgs merge_args(const AttnPlan& p, int heads, const float* part) {
   a.kv_heads = p.kv_heads;
   a.splits1 = p.splits + p.own;
   a.qpad = p.qpad;
-  a.own = p.own;
-  a.run = p.run;
-  a.window = p.window;
   return a;
 }
+
+OwnRuns own_runs(const AttnPlan& p) { return OwnRuns{p.own, p.run, p.window}; }
 
 int block_rows(const AttnPlan& p, int n_q, int b) {
   XTG_CHECK(b >= 0 && b < p.blocks, "attention: block %d of %d", b, p.blocks);
@@ -2184,6 +2477,22 @@ std::string launch_attn_scan(const DevKv& c, const AttnPlan& p, int b0, int nblo
   XTG_CHECK(nblocks >= 1 && b0 + nblocks <= p.blocks, "attention: blocks %d .. %d of %d", b0, b0 + nblocks, p.blocks);
   const int nr = block_rows(p, n_q, b0);   // the widest block of the launch
   const ScanArgs a = scan_args(c, p, b0, q, n_q, heads, pos0, window, scale, part);
+  if (p.quads) {
+    XTG_CHECK(b0 % kWaves == 0, "attention: first block %d", b0);
+    const unsigned wgs = unsigned(c.kv_heads) * unsigned(p.splits) * unsigned((nblocks + kWaves - 1) / kWaves);
+    auto launch = [&](void (*fn)(const ScanArgs, int, int), size_t lds) {
+      allow_lds(reinterpret_cast<const void*>(fn), lds);
+      hipLaunchKernelGGL(fn, dim3(wgs), dim3(2 * kWaves * 64), lds, stream, a, nblocks, c.kv_heads);
+    };
+    if (p.d == 64)
+      launch(c.fp8 ? attn_scan_rows_kernel<64, true> : attn_scan_rows_kernel<64, false>, rows_lds_bytes<64>());
+    else if (p.d == 128)
+      launch(c.fp8 ? attn_scan_rows_kernel<128, true> : attn_scan_rows_kernel<128, false>, rows_lds_bytes<128>());
+    else
+      launch(c.fp8 ? attn_scan_rows_kernel<256, true> : attn_scan_rows_kernel<256, false>, rows_lds_bytes<256>());
+    HIP_CHECK(hipGetLastError());
+    return strf("attn_scan_rows_kernel<%d, %s>", c.head_dim, c.fp8 ? "true" : "false");
+  }
   const int qb = (nr * p.group + 15) / 16;
   ScanFn fn = scan_fn(c.head_dim, qb, c.fp8);
   XTG_CHECK(fn != nullptr, "attention: no kernel for head_dim %d and %d column blocks", c.head_dim, qb);
@@ -2245,11 +2554,11 @@ std::string launch_attn_merge(const AttnPlan& p, int n_q, int heads, const float
                               hipStream_t stream) {
   const MergeArgs a = merge_args(p, heads, part);
   if (p.d == 64)
-    hipLaunchKernelGGL(attn_merge_kernel<64>, dim3(unsigned(n_q)), dim3(kMergeThreads), 0, stream, a, out);
+    hipLaunchKernelGGL(attn_merge_kernel<64>, dim3(unsigned(n_q)), dim3(kMergeThreads), 0, stream, a, own_runs(p), out);
   else if (p.d == 128)
-    hipLaunchKernelGGL(attn_merge_kernel<128>, dim3(unsigned(n_q)), dim3(kMergeThreads), 0, stream, a, out);
+    hipLaunchKernelGGL(attn_merge_kernel<128>, dim3(unsigned(n_q)), dim3(kMergeThreads), 0, stream, a, own_runs(p), out);
   else
-    hipLaunchKernelGGL(attn_merge_kernel<256>, dim3(unsigned(n_q)), dim3(kMergeThreads), 0, stream, a, out);
+    hipLaunchKernelGGL(attn_merge_kernel<256>, dim3(unsigned(n_q)), dim3(kMergeThreads), 0, stream, a, own_runs(p), out);
   HIP_CHECK(hipGetLastError());
   return strf("attn_merge_kernel<%d>", p.d);
 }
@@ -2335,7 +2644,7 @@ std::string launch_attn_gate(const AttnPlan& p, int m, int heads, const float* p
 #define XTG_GATE(D, U)                                                                                      \
   if (p.d == D && chunks <= U * kMergeThreads && !u) {                                                      \
     hipLaunchKernelGGL((attn_gate_kernel<D, U>), grid, block, 0, stream, a, g, gs, vec, out, xop, xinv,    \
-                       op_group_bytes(Q));                                                               \
+                       op_group_bytes(Q), own_runs(p));                                                  \
     u = U;                                                                                                  \
   }
   XTG_GATE(64, 1) XTG_GATE(64, 2) XTG_GATE(64, 4) XTG_GATE(128, 1) XTG_GATE(128, 2) XTG_GATE(128, 4)

@@ -51,12 +51,14 @@ struct AttnPlan {
   int qpad = 16;               // q-cols per block, padded to 16
   int tile_lo = 0, tiles = 0;  // the 32-slot tiles to scan
   int splits = 0;              // work-groups per KV head over the tiles (0: no cached key is visible)
+  bool quads = false;          // the scan's work-groups take 4 row blocks each (attn_scan_rows_kernel)
   int own = 1;                 // own-key records per (block, KV head, q-col), after the splits'
   int run = 32, window = 0;    // own keys per record, the call's window
-  int own_max = 1;             // what scratch is sized for: grows with the rows only, where `own` goes up and down
+  int own_max = 1;             // what scratch is sized for: grows with the rows only, where `own` goes up and down,
+  int splits_max = 0;          // and a ring's as if it were full
   int kv_heads = 1, d = 64;
   size_t records() const { return size_t(blocks) * size_t(kv_heads) * size_t(splits + own) * size_t(qpad); }
-  size_t part_floats() const { return records() / size_t(splits + own) * size_t(splits + own_max) * size_t(d + 2); }
+  size_t part_floats() const { return records() / size_t(splits + own) * size_t(splits_max + own_max) * size_t(d + 2); }
 };
 // fixed_scratch: for the call whose partials go to the fixed array (one own-key record per kOwnChunk keys).
 AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int window, bool fixed_scratch = false);
