@@ -145,8 +145,11 @@ def lib():
     return _lib
 
 
+_ErrBuf = ctypes.c_char * 2048
+
+
 def _errbuf():
-    return ctypes.create_string_buffer(2048)
+    return _ErrBuf()
 
 
 def _check(rc, err):
@@ -165,8 +168,25 @@ def _ptr(a):
     return a.data_ptr()   # torch.Tensor
 
 
+class _Array:
+    """A Weight's array attribute: its address is read when the array is set, not on every call (numpy's .ctypes takes
+    about 0.6 us, three times per weight of a call; a call of four projections spent half of its 14 us there)."""
+
+    def __set_name__(self, owner, name):
+        self.slot = "_" + name
+
+    def __get__(self, w, owner=None):
+        return self if w is None else getattr(w, self.slot)
+
+    def __set__(self, w, a):
+        setattr(w, self.slot, a)
+        setattr(w, self.slot + "_held", a)   # a second reference: numpy then refuses to resize (move) it in place
+        setattr(w, self.slot + "_at", a.ctypes.data)
+
+
 class Weight:
     """An NVFP4 weight held in host memory: codes [n][k/2] u8, scales [n][k/16] u8 (E4M3), global f32."""
+    codes, scales = _Array(), _Array()
 
     def __init__(self, codes, scales, glob=1.0):
         self.codes = np.ascontiguousarray(codes, dtype=np.uint8)
@@ -176,15 +196,19 @@ class Weight:
         self.k = self.codes.shape[1] * 2
         assert self.scales.shape == (self.n_out, self.k // 16)
 
+    def __getstate__(self):   # copies and pickles set their own arrays, and so their own addresses
+        return {"codes": self.codes, "scales": self.scales, "glob": self.glob, "n_out": self.n_out, "k": self.k}
+
+    def __setstate__(self, state):
+        for name, v in state.items():
+            setattr(self, name, v)
+
     def struct(self):
-        return Nvfp4(self.codes.ctypes.data, self.scales.ctypes.data, self.glob, self.n_out, self.k)
+        return Nvfp4(self._codes_at, self._scales_at, self.glob, self.n_out, self.k)
 
 
 def _structs(ws):
-    arr = (Nvfp4 * len(ws))()
-    for i, w in enumerate(ws):
-        arr[i] = w.struct()
-    return arr
+    return (Nvfp4 * len(ws))(*[w.struct() for w in ws])
 
 
 class HipBackend:
@@ -223,7 +247,7 @@ class HipBackend:
 
     def _hold(self, ws):
         for w in ws:
-            self._weights.setdefault(w.codes.ctypes.data, w)
+            self._weights.setdefault(w._codes_at, w)
         return _structs(ws)
 
     def prepare(self, w):
