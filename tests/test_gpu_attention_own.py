@@ -31,6 +31,9 @@ SCANS = [  # heads, kv_heads, head_dim, rows, cached, window, ring slots
     (16, 4, 256, 150, 333, 0, 0), (16, 4, 256, 190, 1400, 1024, 1040), (16, 8, 64, 129, 31, 0, 0),
     (16, 8, 64, 257, 992, 0, 0), (8, 8, 128, 161, 1056, 0, 0), (6, 2, 128, 135, 1100, 0, 0), (10, 2, 256, 128, 95, 64, 0),
     (8, 1, 64, 130, 200, 0, 0),
+    # rings about to wrap and just wrapped, below the rows that share tiles too
+    (32, 8, 128, 20, 700, 500, 1040), (16, 4, 256, 40, 1040, 1024, 1040), (16, 4, 256, 40, 1041, 1000, 1040),
+    (16, 8, 64, 130, 1088, 1024, 1088), (16, 8, 64, 130, 1089, 1024, 1088),
 ]
 
 
