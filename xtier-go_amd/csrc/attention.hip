@@ -1101,7 +1101,7 @@ __global__ void __launch_bounds__(256) attn_own_mfma_kernel(const OwnArgs a) {
 // Waves per SIMD: one at 64 and 128 dims and two work-groups a CU; at 256 dims two waves share a row block
 // (own_halves), one work-group a CU. LDS reads take half of the matrix ops' time (each operand read feeds two column
 // blocks: with one a wave they would take all of it). Measured (512 rows, no cached keys, in the kernel): 16 / 4 heads
-// of 256, 107 us with the FP32 kernel, 38 us here; 32 / 8 of 128, 51 and 27 us. The matrix ops are busy for a fifth of
+// of 256, 107 us with the FP32 kernel, 41 us here (38 in runs of 128 keys); 32 / 8 of 128, 51 and 28 us. The matrix ops are busy for a fifth of
 // that: a run is 3-4 tiles long, each 3-4 us of scores 1.1, softmax and splits 0.7, outputs 1.4 and barriers 0.8 in a
 // chain, after about 4 us of first loads and of code that is fetched the first time.
 
