@@ -102,3 +102,32 @@ def test_an_infinite_value_stays_infinite(hip):
     cache.destroy()
     assert (got[at:, 0, 3] == np.inf).all()
     assert np.isfinite(got[:at // 32 * 32]).all() and np.isfinite(got[:, 1:]).all()
+
+
+@pytest.mark.parametrize("heads,kv,d,n,window,ats", [
+    (4, 4, 128, 160, 0, (100, 159)), (32, 8, 128, 150, 0, (31, 32, 149)), (16, 4, 256, 70, 20, (0, 40, 69)),
+    (8, 1, 64, 131, 50, (64, 65, 130))])
+def test_rows_that_do_not_see_a_value_stay_finite(hip, heads, kv, d, n, window, ats):
+    """Infinities and a NaN in V: the rows that see their key have them, every other row and dim is bit for bit what it
+    is with zeros in their place."""
+    rng = np.random.default_rng(n)
+    q, k, v = (rng.standard_normal((n, h, d)).astype(np.float32) * 0.1 for h in (heads, kv, kv))
+    odd = [(at, i % kv, 3 + 29 * i, x) for i, at in enumerate(ats) for x in ((np.inf, -np.inf, np.nan)[i],)]
+    cache = hip.kv_cache(kv, d, n)
+    out = hip.array(np.zeros((n, heads, d), np.float32))
+
+    def call(v):
+        hip.attention(cache, hip.array(q), hip.array(k), hip.array(v), out, n, 0, heads, window)
+        return out.numpy().reshape(n, heads, d).copy()
+
+    for at, h, dim, _ in odd:
+        v[at, h, dim] = 0
+    want = call(v)
+    assert np.isfinite(want).all()
+    for at, h, dim, x in odd:
+        v[at, h, dim] = x
+        for row in range(at, min(n, at + window) if window else n):
+            want[row, h * (heads // kv):(h + 1) * (heads // kv), dim] = x
+    got = call(v)
+    cache.destroy()
+    np.testing.assert_array_equal(got, want)

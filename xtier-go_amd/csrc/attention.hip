@@ -1159,10 +1159,11 @@ __device__ __forceinline__ void pace_reads() {
 // exchanged through LDS, and its half of the outputs), so that two waves fit a SIMD.
 template <int D>
 constexpr int own_halves() { return D == 256 ? 2 : 1; }
-// K and V terms of one tile, and the exchanged score sums (16 floats a lane).
+// K and V terms of one tile, the exchanged score sums (16 floats a lane), and a flag per wave.
 template <int D>
 constexpr size_t own_lds_bytes() {
-  return size_t(2 * kTile) * D * 3 * 2 + (own_halves<D>() == 2 ? size_t(2 * kWaves) * 16 * 64 * sizeof(float) : 0);
+  return size_t(2 * kTile) * D * 3 * 2 + (own_halves<D>() == 2 ? size_t(2 * kWaves) * 16 * 64 * sizeof(float) : 0) +
+         2 * kWaves * sizeof(int);
 }
 // A column's running maximum is moved only when a score exceeds it by more than this many powers of two: weights and
 // sums stay below 2^8 times what they would be, and most tiles need no maximum over lanes and no rescaling.
@@ -1177,6 +1178,7 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
   bf16x8* const lk = reinterpret_cast<bf16x8*>(own_lds);
   bf16x8* const lv = lk + 2 * NC * 3 * 64;
   f32x4* const ex = reinterpret_cast<f32x4*>(lv + ND * 3 * 64);
+  int* const odd_v = reinterpret_cast<int*>(ex + (H == 2 ? W * 4 * 64 : 0));   // [W]: the wave staged a V that is not finite
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int rb = wave % kWaves, h = wave / kWaves;
   const int g = lane >> 4, j = lane & 15;
@@ -1231,14 +1233,26 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
       for (int n = 0; n < 3; ++n) lk[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
     }
   };
+  // V that is not finite goes in as zeros and is added after the last tile: in the matrix ops it would meet the weight 0
+  // of the columns that do not see its key, and make NaN of it
+  bool odd = false;
   auto put_v = [&](const float (&st)[VU][8]) {
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const bool finite = __builtin_fabsf(st[u][e]) < INFINITY;
+        x[e] = finite ? st[u][e] : 0.f;
+        odd |= !finite;
+      }
       bf16x8 t[3];
-      split_exact<true>(st[u], t);
+      split_exact<false>(x, t);
 #pragma unroll
       for (int n = 0; n < 3; ++n) lv[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
     }
+    odd = __ballot(odd) != 0;
+    if (lane == 0) odd_v[wave] = odd;
   };
   static_assert(KU == VU, "one staging array");
   float st[KU][8];   // the next tile's K until the scores are done, then its V
@@ -1375,6 +1389,27 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
     }
     __syncthreads();   // V (and the halves' sums) read by every wave, the next K complete
     if (more) put_v(st);
+  }
+
+  // what of V is not finite, for the columns that see its key. Any weight above 0 gives the same infinity or NaN; a
+  // weight that has fallen below FP32's range counts as above 0, too.
+  int any_odd = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) any_odd |= odd_v[w];
+  if (__builtin_amdgcn_readfirstlane(any_odd)) {
+    for (int key = max(kmin, first_any); key < kmax && key <= i_last; ++key) {
+      const float* vr = a.v + (size_t(key) * a.kv_heads + size_t(kvh)) * D + 16 * h * NDH + 4 * g;
+#pragma unroll
+      for (int dd = 0; dd < NDH; ++dd) {
+        const float4 x4 = *reinterpret_cast<const float4*>(vr + 16 * dd);
+        const float x[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb)
+            if (!(__builtin_fabsf(x[r]) < INFINITY) && key >= lo[qb] && key <= hi[qb]) o[qb][dd][r] += x[r];
+      }
+    }
   }
 
 #pragma unroll
