@@ -3,7 +3,7 @@ rows where it takes over from the few-row kernel, ragged tiles and runs, windows
 not fill a row block, and every head size, against FP64.
 
 Bar: max |err| / RMS <= 3e-5. A score of magnitude 8 (in powers of two) is off by at most about 8 * 2^-22 after D
-FP32 additions of products good to 2^-23, so a weight by 1.4e-6 of itself; an output adds up as many of those as keys
+FP32 additions of products good to 2^-24, so a weight by 1.4e-6 of itself; an output adds up as many of those as keys
 carry weight, and its own rounding, against an RMS that falls with the number of keys averaged: 1e-5 was the largest
 measured at 1500 rows."""
 import numpy as np
@@ -131,3 +131,62 @@ def test_rows_that_do_not_see_a_value_stay_finite(hip, heads, kv, d, n, window, 
     got = call(v)
     cache.destroy()
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("bits", [0x3f80ffff, 0x3f807fc0, 0x3fd5a5a5])
+@pytest.mark.parametrize("heads,kv,d,n", [(4, 4, 64, 70), (2, 2, 128, 100), (2, 2, 256, 70)])
+def test_products_of_scores_keep_their_bits(hip, heads, kv, d, n, bits):
+    """Scores that are sums of d products of 64 which cancel, so that the sums' roundings vanish and what is left out of
+    the products shows: half of them of two values with full mantissas, half of one and its BF16 rounding (whose products
+    are whole). Bar: d / 2 products of |x y| each short of at most 2^-24 + 2^-34 of it, times ln 2, and 1e-5 of the
+    weight for the other roundings."""
+    scale = next(s for s in np.nextafter(np.float32(np.log(2)), np.float32([0, 1, 0.69314718])) if
+                 np.float32(s) * np.float32(1.44269504088896341) == 1)   # scores in powers of two, as they are
+    x = np.uint32(bits).view(np.float32)
+    xb = np.uint32((bits + 0x7fff + ((bits >> 16) & 1)) & 0xffff0000).view(np.float32)
+    q = np.full((n, heads, d), x * 64 / np.exp2(np.floor(np.log2(x * x))), np.float32)
+    k, v = np.zeros((n, kv, d), np.float32), np.zeros((n, kv, d), np.float32)
+    k[0, :, 0::2], k[0, :, 1::2] = x, -xb
+    k[1, :, 0::2] = ((x - xb).view(np.uint32) & np.uint32(0xffff0000)).view(np.float32)   # about its score, whole
+    v[0] = 1
+    w = np.exp2(q[0, 0].astype(np.float64) @ k[:, 0].T.astype(np.float64))
+    exact = w[0] / np.cumsum(w)
+    cache = hip.kv_cache(kv, d, n)
+    out = hip.array(np.zeros((n, heads, d), np.float32))
+    hip.attention(cache, hip.array(q), hip.array(k), hip.array(v), out, n, 0, heads, 0, float(scale))
+    got = out.numpy().reshape(n, heads, d).astype(np.float64)
+    cache.destroy()
+    short = d / 2 * float(q[0, 0, 0]) * float(x) * (2.0 ** -24 + 2.0 ** -34)
+    err = np.max(np.abs(got - exact[:, None, None]) / exact[:, None, None])
+    assert err <= short * np.log(2) + 1e-5, (err, short)
+
+
+@pytest.mark.parametrize("d,n", [(64, 70), (128, 70), (256, 70)])
+def test_values_at_the_ends_of_the_range(hip, d, n):
+    """FP32's largest value in V (BF16 would round it to infinity), minus infinity in K (a weight of 0 for these q, all
+    above 0), and a NaN whose bits are all in the lower half, which its row and the later ones show. Bar: 3e-5 of the
+    value, as above (6 keys' worth of relative weight errors at most)."""
+    heads = 2
+    rng = np.random.default_rng(d)
+    q = rng.uniform(0.5, 1, (n, heads, d)).astype(np.float32)
+    k, v = (rng.standard_normal((n, heads, d)).astype(np.float32) * 0.1 for _ in range(2))
+    k[10, :, 5] = -np.inf
+    k[60, 1, 7] = np.uint32(0x7f800001).view(np.float32)
+    v[30, 0, 2] = np.finfo(np.float32).max
+    cache = hip.kv_cache(heads, d, n)
+    out = hip.array(np.zeros((n, heads, d), np.float32))
+    hip.attention(cache, hip.array(q), hip.array(k), hip.array(v), out, n, 0, heads, 0)
+    got = out.numpy().reshape(n, heads, d).astype(np.float64)
+    cache.destroy()
+    assert np.isnan(got[60:, 1]).all()
+    k[60, 1] = 0   # of no row below
+    for h in range(heads):
+        s = q[:, h].astype(np.float64) @ k[:, h].astype(np.float64).T / np.sqrt(d)
+        s[np.arange(n)[None, :] > np.arange(n)[:, None]] = -np.inf
+        s[:, 10] = -np.inf
+        rows = n if h == 0 else 60
+        p = np.exp(s[:rows] - s[:rows].max(axis=1, keepdims=True))
+        exact = (p / p.sum(axis=1, keepdims=True)) @ v[:, h].astype(np.float64)
+        assert np.isfinite(got[:rows, h]).all()
+        scale = np.where(np.abs(exact) > 1, np.abs(exact), 0.02)   # the other values' size
+        assert np.max(np.abs(got[:rows, h] - exact) / scale) <= 3e-5

@@ -1088,9 +1088,10 @@ __global__ void __launch_bounds__(256) attn_own_mfma_kernel(const OwnArgs a) {
 }
 
 // Own keys on the matrix cores, for calls of many rows. FP32 rows go through v_mfma_f32_16x16x32_bf16 in three exact
-// BF16 terms each (split_exact: 24 bits = 3 x 8): of the nine products of two such values the six down to 2^-16 are
-// taken, what is dropped is below 2^-23 of the product, and sums are FP32. That is 6 matrix ops of 16 cycles for what
-// v_mfma_f32_16x16x4_f32 takes 8 of 32 cycles for.
+// BF16 terms each (split_exact: 24 bits = 3 x 8): of the nine products of two such values the six down to 2^-17 are
+// taken, what is dropped (t1 u2 + t2 u1 + t2 u2) is at most 2^-24 + 2^-34 of the product, the half unit that an FP32
+// product is rounded by, and sums are FP32. That is 6 matrix ops of 16 cycles for what v_mfma_f32_16x16x4_f32 takes 8 of
+// 32 cycles for.
 //
 // A work-group of 4 waves takes 4 consecutive row blocks (a wave each, its 2 x 16 q-cols) of one KV head and one of
 // `own` runs of keys, in tiles of 32 keys whose K and V the 4 waves share: each wave loads a quarter of a tile as FP32
@@ -1105,31 +1106,56 @@ __global__ void __launch_bounds__(256) attn_own_mfma_kernel(const OwnArgs a) {
 // that: a run is 3-4 tiles long, each 3-4 us of scores 1.1, softmax and splits 0.7, outputs 1.4 and barriers 0.8 in a
 // chain, after about 4 us of first loads and of code that is fetched the first time.
 
-// x = t0 + t1 + t2 exactly: each term the upper half of what is left (8 bits of the 24). ANY: an infinity or a NaN
-// comes as the last term alone, which meets the other operand's first term only (as the first it would meet second and
-// third terms that are zero, and make NaN of an infinity). Without ANY, x is finite or NaN.
-__device__ inline uint32_t upper_halves(float lo, float hi) {
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+// x = t0 + t1 + t2 exactly: each term the BF16 rounding of what is left (8 bits of the 24), so that |t1| <= 2^-8 |x|,
+// |t2| <= 2^-17 |x|, and either sign is as likely. ANY: an infinity or a NaN comes as the last term alone, which meets
+// the other operand's first term only (as the first it would meet second and third terms that are zero, and make NaN of
+// an infinity), and a value that would round to infinity has kBf16Max as its first term. Without ANY, x is a NaN or at
+// most kBf16Max.
+constexpr float kBf16Max = 0x1.fep127f;
+__device__ inline uint32_t bf16_pair(float lo, float hi) {   // v_cvt_pk_bf16_f32
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 template <bool ANY>
 __device__ inline void split_exact(const float (&v)[8], bf16x8 (&t)[3]) {
-  float x[8], r1[8], r2[8];
+  uint32_t u[3][4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float x[2], r[2];
+    bool finite[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      finite[i] = !ANY || __builtin_fabsf(v[2 * e + i]) < INFINITY;
+      x[i] = finite[i] ? v[2 * e + i] : 0.f;
+      r[i] = ANY ? __builtin_amdgcn_fmed3f(x[i], -kBf16Max, kBf16Max) : x[i];
+    }
+    u[0][e] = bf16_pair(r[0], r[1]);
+    r[0] = x[0] - __uint_as_float(u[0][e] << 16);
+    r[1] = x[1] - __uint_as_float(u[0][e] & 0xffff0000u);
+    u[1][e] = bf16_pair(r[0], r[1]);
+    r[0] -= __uint_as_float(u[1][e] << 16);
+    r[1] -= __uint_as_float(u[1][e] & 0xffff0000u);
+    // what is left has 8 bits: its upper half is all of it (v + v: a NaN whose bits are all in the lower half, made quiet)
+    u[2][e] = __builtin_amdgcn_perm(__float_as_uint(finite[1] ? r[1] : v[2 * e + 1] + v[2 * e + 1]),
+                                    __float_as_uint(finite[0] ? r[0] : v[2 * e] + v[2 * e]), 0x07060302u);
+  }
+#pragma unroll
+  for (int n = 0; n < 3; ++n) t[n] = __builtin_bit_cast(bf16x8, make_uint4(u[n][0], u[n][1], u[n][2], u[n][3]));
+}
+
+// Whether some lane's values (or their sum) are not below kBf16Max, NaN among them: the rare case of a tile.
+template <int N>
+__device__ inline bool some_large(const float (&v)[N][8]) {
+  float s[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const bool finite = !ANY || __builtin_fabsf(v[e]) < INFINITY;
-    x[e] = finite ? v[e] : 0.f;
-    r1[e] = x[e] - __uint_as_float(__float_as_uint(x[e]) & 0xffff0000u);
-    r2[e] = r1[e] - __uint_as_float(__float_as_uint(r1[e]) & 0xffff0000u);
-    if (!finite) r2[e] = v[e];
-  }
-  uint4 u[3];
-  u[0] = make_uint4(upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7]));
-  u[1] = make_uint4(upper_halves(r1[0], r1[1]), upper_halves(r1[2], r1[3]), upper_halves(r1[4], r1[5]),
-                    upper_halves(r1[6], r1[7]));
-  u[2] = make_uint4(upper_halves(r2[0], r2[1]), upper_halves(r2[2], r2[3]), upper_halves(r2[4], r2[5]),
-                    upper_halves(r2[6], r2[7]));
+    s[e] = __builtin_fabsf(v[0][e]);
 #pragma unroll
-  for (int n = 0; n < 3; ++n) t[n] = __builtin_bit_cast(bf16x8, u[n]);
+    for (int n = 1; n < N; ++n) s[e] += __builtin_fabsf(v[n][e]);
+  }
+  const float sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  return __builtin_expect(__ballot(!(sum < kBf16Max)) != 0, 0);
 }
 
 // The six products of A = a0 + a1 + a2 and B = b0 + b1 + b2, smallest first, onto one accumulator per column block.
@@ -1225,10 +1251,14 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
     }
   };
   auto put_k = [&](const float (&st)[KU][8]) {
+    const bool large = some_large(st);
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       bf16x8 t[3];
-      split_exact<true>(st[u], t);
+      if (large)
+        split_exact<true>(st[u], t);
+      else
+        split_exact<false>(st[u], t);
 #pragma unroll
       for (int n = 0; n < 3; ++n) lk[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
     }
@@ -1237,17 +1267,22 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
   // of the columns that do not see its key, and make NaN of it
   bool odd = false;
   auto put_v = [&](const float (&st)[VU][8]) {
+    const bool large = some_large(st);
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
-      float x[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const bool finite = __builtin_fabsf(st[u][e]) < INFINITY;
-        x[e] = finite ? st[u][e] : 0.f;
-        odd |= !finite;
-      }
       bf16x8 t[3];
-      split_exact<false>(x, t);
+      if (large) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const bool finite = __builtin_fabsf(st[u][e]) < INFINITY;
+          x[e] = finite ? st[u][e] : 0.f;
+          odd |= !finite;
+        }
+        split_exact<true>(x, t);
+      } else {
+        split_exact<false>(st[u], t);
+      }
 #pragma unroll
       for (int n = 0; n < 3; ++n) lv[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
     }
