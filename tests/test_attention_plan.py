@@ -1,0 +1,63 @@
+"""The host-side plan of an attention call (attn_plan in csrc/attention.hip), through the library without a GPU: the
+scratch it asks for covers its records, is the same at every position of a cache (a prompt's later chunk, or a graph
+captured after an early call, must not outgrow it)."""
+import collections
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#include <cstdio>
+#include "attention.hpp"
+int main() {
+  xtg::hip::DevKv c;
+  int n_q, heads, window, fixed, ring, fp8;
+  long long pos0;
+  while (std::scanf("%d %d %lld %d %d %d %d %lld %d %d", &c.kv_heads, &c.head_dim, &c.slots, &ring, &fp8, &n_q, &heads,
+                    &pos0, &window, &fixed) == 10) {
+    c.ring = ring, c.fp8 = fp8, c.slots_pad = int((c.slots + 31) / 32 * 32);
+    const xtg::hip::AttnPlan p = xtg::hip::attn_plan(c, n_q, heads, pos0, window, fixed != 0);
+    std::printf("%d %d %d %d %d %zu %zu\n", p.tiles, p.splits, int(p.quads), p.own, p.run, p.records() * (p.d + 2),
+                p.part_floats());
+  }
+}
+"""
+Plan = collections.namedtuple("Plan", "tiles splits shared own run used floats")
+
+
+@pytest.fixture(scope="module")
+def plans(pkg, tmp_path_factory):
+    """plans([(kv_heads, head_dim, slots, ring, fp8, n_q, heads, pos0, window, fixed)]) -> [Plan]"""
+    d = tmp_path_factory.mktemp("plan")
+    (d / "plan.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "xtier-go_amd", "csrc"), str(d / "plan.cpp"), pkg.LIB_PATH,
+                    "-Wl,-rpath," + os.path.dirname(pkg.LIB_PATH), "-L/opt/rocm/lib", "-lamdhip64", "-o",
+                    str(d / "plan")], check=True)
+
+    def run(calls):
+        text = "\n".join(" ".join(str(int(v)) for v in c) for c in calls) + "\n"
+        env = {k: v for k, v in os.environ.items() if not k.startswith("XTG_")}
+        r = subprocess.run([str(d / "plan")], input=text, capture_output=True, text=True, check=True, env=env)
+        out = [Plan(*map(int, line.split())) for line in r.stdout.splitlines()]
+        assert len(out) == len(calls)
+        return out
+
+    return run
+
+
+@pytest.mark.parametrize("heads,kv,d", [(32, 8, 128), (16, 4, 256), (16, 8, 64), (8, 8, 128), (2, 1, 128), (64, 8, 256)])
+@pytest.mark.parametrize("slots,ring,window", [(1040, 1, 1024), (1088, 1, 1024), (700, 1, 0), (9000, 0, 0), (9000, 0, 1024)])
+def test_scratch_is_the_same_at_every_position(plans, heads, kv, d, slots, ring, window):
+    for n_q in (1, 8, 20, 48, 130, 188, 512):
+        last = 3 * slots if ring else slots - n_q
+        if last < 0:
+            continue
+        at = sorted({0, 1, 31, 33, 512, 1000, 1023, 1024, 1025, slots // 2, slots - 1, slots, slots + 1, last} & set(range(last + 1)))
+        for fp8 in (0, 1):
+            ps = plans([(kv, d, slots, ring, fp8, n_q, heads, pos, window, 0) for pos in at])
+            assert len({p.floats for p in ps}) == 1, (n_q, list(zip(at, ps)))
+            assert all(p.used <= p.floats and p.splits <= p.tiles for p in ps)

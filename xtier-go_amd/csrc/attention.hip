@@ -2301,29 +2301,30 @@ AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int windo
   // 8 %, and 512 work-groups take 1.5 % off the one-token step at 32K (1.099 -> 1.082 ms, with the gate's merge on
   // more waves; 0.2 % at 8K; 768 and 1024: 1.109 and 1.105 ms), while at 8 rows they cost 4 %.
   // (XTG_ATTN_SPLITS=n fixes the count, for experiments)
+  // Calls of many rows share their tiles (attn_scan_rows_kernel), a work-group per CU with at least 4 tiles each. Whole
+  // calls, each on its own tiles and shared: 64 rows over 1500 keys 29.9 and 36 us (128 dims), 47.6 and 55 us (256); 96
+  // rows 36.6 and 37.9; 128 rows 48 and 43 us, 77 and 54 us; 128 dims and few tiles, 256 rows over 300 keys, 40 and 43
+  // us, where 256 dims take 71 and 58 us. (The fixed array's calls keep the plan that fits it.)
+  auto shared = [&](int tiles) { return !fixed_scratch && n_q >= 128 && (c.head_dim != 128 || tiles >= 32); };
+  const char* const env = std::getenv("XTG_ATTN_SPLITS");
   auto splits_of = [&](int tiles) {
+    if (tiles == 0) return 0;
     const int wgs = c.fp8 && !c.ring && n_q == 1 ? 512 : 192;
     const int want = std::max(1, wgs / (c.kv_heads * p.blocks));   // about wgs work-groups over all blocks
     const int mt = c.ring ? 1 : 2;
-    int n = std::max(1, std::min(want, (tiles + mt * kWaves - 1) / (mt * kWaves)));
-    if (const char* env = std::getenv("XTG_ATTN_SPLITS")) n = std::max(1, std::atoi(env));
-    return std::min(n, tiles);
-  };
-  if (p.tiles > 0) {
-    p.splits = splits_of(p.tiles);
-    // calls of many rows share their tiles (attn_scan_rows_kernel), a work-group per CU with at least 4 tiles each.
-    // Whole calls, each on its own tiles and shared: 64 rows over 1500 keys 29.9 and 36 us (128 dims), 47.6 and 55 us
-    // (256); 96 rows 36.6 and 37.9; 128 rows 48 and 43 us, 77 and 54 us; 128 dims and few tiles, 256 rows over 300
-    // keys, 40 and 43 us, where 256 dims take 71 and 58 us. (The fixed array's calls keep the plan that fits it.)
     const int quads = c.kv_heads * ((p.blocks + kWaves - 1) / kWaves);
-    p.quads = !fixed_scratch && n_q >= 128 && (c.head_dim != 128 || p.tiles >= 32);
-    if (p.quads && !std::getenv("XTG_ATTN_SPLITS")) {
-      p.splits = std::max(1, std::min(256 / quads, p.tiles / 4));
-    }
-  } else {
-    p.splits = 0;
-  }
-  p.splits_max = c.ring ? std::max(p.splits, splits_of(ring_tiles)) : p.splits;
+    int n = env ? std::atoi(env)
+                : shared(tiles) ? std::min(256 / quads, tiles / 4)
+                                : std::min(want, (tiles + mt * kWaves - 1) / (mt * kWaves));
+    return std::min(std::max(1, n), tiles);
+  };
+  p.splits = splits_of(p.tiles);
+  p.quads = p.tiles > 0 && shared(p.tiles);
+  // Scratch holds the most splits of any position, so that no later call of as many rows outgrows it (in the middle of a
+  // prompt, or in a graph capture): more tiles never get fewer splits, but for where tiles begin to be shared. The
+  // allocation-free call checks its own need, on a ring that of a full one.
+  p.splits_max = p.splits;
+  if (c.ring || !fixed_scratch) p.splits_max = std::max(splits_of(ring_tiles), splits_of(std::min(ring_tiles, 31)));
   plan_own(p, n_q, window, fixed_scratch);
   return p;
 }

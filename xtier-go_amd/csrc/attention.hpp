@@ -54,8 +54,8 @@ struct AttnPlan {
   bool quads = false;          // the scan's work-groups take 4 row blocks each (attn_scan_rows_kernel)
   int own = 1;                 // own-key records per (block, KV head, q-col), after the splits'
   int run = 32, window = 0;    // own keys per record, the call's window
-  int own_max = 1;             // what scratch is sized for: grows with the rows only, where `own` goes up and down,
-  int splits_max = 0;          // and a ring's as if it were full
+  int own_max = 1;             // what scratch is sized for: the most records of any position in this cache,
+  int splits_max = 0;          // whatever this call's
   int kv_heads = 1, d = 64;
   size_t records() const { return size_t(blocks) * size_t(kv_heads) * size_t(splits + own) * size_t(qpad); }
   size_t part_floats() const { return records() / size_t(splits + own) * size_t(splits_max + own_max) * size_t(d + 2); }
