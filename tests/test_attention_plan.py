@@ -61,3 +61,14 @@ def test_scratch_is_the_same_at_every_position(plans, heads, kv, d, slots, ring,
             ps = plans([(kv, d, slots, ring, fp8, n_q, heads, pos, window, 0) for pos in at])
             assert len({p.floats for p in ps}) == 1, (n_q, list(zip(at, ps)))
             assert all(p.used <= p.floats and p.splits <= p.tiles for p in ps)
+
+
+def test_the_allocation_free_call_needs_what_it_writes(plans):
+    """One own-key record per 128 keys and the splits of a full cache, whichever kernel takes the own keys: 48 rows of 256
+    heads of 128 over 32 KV heads fit the 16 MiB array with one split."""
+    calls = [(32, 128, 4096, 0, 0, 48, 256, 2000, 0, 1)]
+    calls += [(kv, d, 1040, 1, 0, n, kv * group, 3000, 1024, 1) for d in (64, 128, 256) for kv, group in ((8, 4), (2, 8), (4, 1))
+              for n in (1, 8, 9, 33, 48, 49, 100, 128, 129, 250)]
+    for call, p in zip(calls, plans(calls)):
+        assert p.used == p.floats and p.own == -(-call[5] // 128), (call, p)
+    assert plans(calls[:1])[0].floats * 4 == 32 * 12 * 2 * 32 * 130 * 4 < 16 << 20

@@ -6,11 +6,14 @@ the C ABI. Bar: equal bit for bit (integer-exact agreement is expected: the same
   ring read by one row), so the second runs on what the first left in the shared array; FP8 caches as well.
 - A fresh backend, whose own attention scratch was never sized, captures the call into a HIP graph and replays it
   (first in this file: the array then belongs to that backend until it is closed).
+- Calls of many rows whose own keys take one and several records of 128 keys, against FP64.
 - A call whose partials exceed the array is refused before anything is queued; so is a call from a second open
   backend on the device while the first holds the array (their calls would race on it).
 """
 import numpy as np
 import pytest
+
+from test_gpu_attention_own import run as own_keys
 
 pytestmark = pytest.mark.gpu
 
@@ -82,6 +85,15 @@ def test_noalloc_matches_attention_two_calls(hip, dtype):
         cache.destroy()
         for a in arrays:
             a.free()
+
+
+@pytest.mark.parametrize("heads,kv,d,n,cached,window", [
+    (256, 32, 128, 48, 300, 0), (64, 8, 128, 150, 0, 0), (64, 8, 128, 150, 70, 100), (64, 8, 128, 100, 300, 0),
+    (32, 8, 64, 200, 0, 0), (32, 8, 64, 40, 1000, 500), (64, 8, 256, 66, 0, 0), (8, 8, 128, 190, 700, 0)])
+def test_noalloc_many_rows(hip, pkg, heads, kv, d, n, cached, window):
+    """Bars of test_gpu_attention_own.py."""
+    err = own_keys(hip, pkg, heads, kv, d, n, cached, window, call=hip.attention_noalloc)
+    assert err <= (6e-5 if cached else 3e-5), err
 
 
 def test_noalloc_refuses_more_than_its_scratch(hip, pkg):

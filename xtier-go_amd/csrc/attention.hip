@@ -2219,12 +2219,12 @@ void plan_own(AttnPlan& p, int n_q, int window, bool fixed_scratch) {
   // the keys a work-group's rows see, from a multiple of the tile on
   const long long range = window > 0 ? std::min<long long>(n_q, (long long)window + rows + kTile - 2) : n_q;
   const int tiles = int((range + kTile - 1) / kTile);
-  p.own_max = std::max(fixed, std::min(8, tiles));
   if (own_few_rows(p.d, n_q)) {
-    p.own = 1;
+    p.own = p.own_max = 1;
     p.run = tiles * kTile;
     return;
   }
+  p.own_max = std::max(fixed, std::min(8, tiles));
   if (fixed_scratch) {
     p.own = p.own_max = fixed;
     p.run = (tiles + fixed - 1) / fixed * kTile;
