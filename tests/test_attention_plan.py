@@ -1,6 +1,6 @@
 """The host-side plan of an attention call (attn_plan in csrc/attention.hip), through the library without a GPU: the
 scratch it asks for covers its records, is the same at every position of a cache (a prompt's later chunk, or a graph
-captured after an early call, must not outgrow it)."""
+captured after an early call, must not outgrow it), and calls take the kernel that measured faster."""
 import collections
 import os
 import subprocess
@@ -20,12 +20,12 @@ int main() {
                     &pos0, &window, &fixed) == 10) {
     c.ring = ring, c.fp8 = fp8, c.slots_pad = int((c.slots + 31) / 32 * 32);
     const xtg::hip::AttnPlan p = xtg::hip::attn_plan(c, n_q, heads, pos0, window, fixed != 0);
-    std::printf("%d %d %d %d %d %zu %zu\n", p.tiles, p.splits, int(p.quads), p.own, p.run, p.records() * (p.d + 2),
+    std::printf("%d %d %d %d %d %d %zu %zu\n", p.tiles, p.splits, int(p.quads), int(p.few), p.own, p.run, p.records() * (p.d + 2),
                 p.part_floats());
   }
 }
 """
-Plan = collections.namedtuple("Plan", "tiles splits shared own run used floats")
+Plan = collections.namedtuple("Plan", "tiles splits shared few own run used floats")
 
 
 @pytest.fixture(scope="module")
@@ -72,3 +72,13 @@ def test_the_allocation_free_call_needs_what_it_writes(plans):
     for call, p in zip(calls, plans(calls)):
         assert p.used == p.floats and p.own == -(-call[5] // 128), (call, p)
     assert plans(calls[:1])[0].floats * 4 == 32 * 12 * 2 * 32 * 130 * 4 < 16 << 20
+
+
+@pytest.mark.parametrize("heads,kv,d,last", [
+    (16, 8, 64, 48), (8, 1, 64, 48), (32, 32, 64, 48), (8, 8, 128, 48), (2, 1, 128, 52), (32, 8, 128, 52), (64, 8, 128, 52),
+    (4, 4, 256, 20), (8, 4, 256, 28), (16, 4, 256, 36), (8, 1, 256, 33)])
+def test_calls_of_few_rows_keep_the_few_row_kernel(plans, heads, kv, d, last):
+    """Up to the last rows at which it measured no slower than the tiled kernel."""
+    for window in (0, 1024):
+        ps = plans([(kv, d, 1040, 1, 0, n, heads, 500, window, 0) for n in (9, last, last + 1)])
+        assert [p.few for p in ps] == [1, 1, 0] and ps[0].own == ps[1].own == 1

@@ -19,6 +19,10 @@ CASES = [  # heads, kv_heads, head_dim, rows, cached, window
     (8, 1, 64, 67, 0, 0),        # eight: 4-row blocks
     (6, 2, 128, 75, 0, 0),       # three: 10-row blocks of 30 columns
     (10, 2, 256, 61, 0, 0),      # five: 6-row blocks of 30 columns
+    # the rows on either side of the few-row kernel, at each size of group
+    (16, 8, 64, 48, 0, 0), (16, 8, 64, 49, 0, 0), (8, 1, 64, 48, 20, 30), (8, 8, 128, 48, 0, 0), (8, 8, 128, 49, 0, 0),
+    (32, 8, 128, 52, 0, 0), (32, 8, 128, 53, 0, 0), (4, 4, 256, 20, 0, 0), (4, 4, 256, 21, 0, 0), (8, 4, 256, 28, 0, 0),
+    (8, 4, 256, 29, 0, 0), (16, 4, 256, 36, 0, 0), (16, 4, 256, 37, 0, 0), (8, 1, 256, 33, 0, 0), (8, 1, 256, 34, 0, 0),
     (32, 8, 128, 300, 0, 100), (16, 4, 256, 200, 0, 33), (16, 8, 64, 400, 0, 1), (32, 8, 128, 530, 40, 500),
 ]
 

@@ -977,7 +977,7 @@ struct OwnArgs {
   float scale2;
 };
 
-// Own keys on the matrix cores, for calls of few rows (own_few_rows): FP32 MFMA 16x16x4, one wave per tile of 16
+// Own keys on the matrix cores, for calls of few rows (AttnPlan::few): FP32 MFMA 16x16x4, one wave per tile of 16
 // q-cols of a row block over all the keys that any of its columns sees, 16 keys a step, one record. What bounds such a
 // call is one wave's chain of loads and the code it runs once, so nothing is staged or shared:
 //   S^T (16 keys x 16 q-cols) = K Q^T: at step s lane group g (lane / 16) feeds dim (D / 4) g + s of key / q-col
@@ -2197,10 +2197,18 @@ __global__ void __launch_bounds__(64 * W) attn_merge_heads_kernel(const MergeArg
 
 namespace {
 
-// Calls of few rows keep the FP32 kernel, whose waves share nothing and wait for nothing. Whole attention calls, that
-// kernel and the tiled one: 32 rows of 128 dims 10.7 and 13.0 us, 48: 12.5 and 13.2, 64: 14.8 and 13.3; 24 rows of 256
-// dims 17.0 and 17.4, 40: 21.4 and 19.3; 64-dim heads are equal up to 40 rows and the tiled kernel faster above.
-bool own_few_rows(int d, int n_q) { return n_q <= (d == 128 ? 48 : d == 256 ? 32 : 0); }
+// Calls of few rows keep the FP32 kernel, whose waves share nothing and wait for nothing. Both kernels' time goes with
+// the rows (the keys of the longest chain) and hardly with the KV heads; the FP32 kernel's also with the columns that a
+// row block's rows fill, so with the group. On the GPU, own keys and merge, that kernel and the tiled one (21 pairs of
+// heads and sizes, 9 to 128 rows): 16 / 8 heads of 64, 9 rows 6.3 and 7.9 us, 48: 8.8 and 8.8, 64: 9.8 and 9.2; 32 / 8
+// of 128, 48: 12.4 and 13.4, 52: 12.4 and 13.5, 56: 13.8 and 13.6; 8 / 8 of 128, 48: 10.2 and 11.2, 49: 12.6 and 11.3; 4 / 4
+// of 256, 16: 12.6 and 14.1, 24: 15.7 and 14.7; 8 / 4 of 256, 28: 16.0 and 16.0; 16 / 4 of 256, 36: 18.9 and 19.3, 40: 21.5
+// and 19.4; 8 / 1 of 256, 33: 18.6 and 19.0, 36: 20.4 and 19.1.
+bool own_few_rows(int d, int group, int n_q) {
+  if (d == 64) return n_q <= 48;
+  if (d == 128) return n_q <= (group == 1 ? 48 : 52);
+  return n_q <= (group == 1 ? 20 : group == 2 ? 28 : group <= 4 ? 36 : 33);
+}
 
 // The runs of own keys: a work-group of attn_own_kernel (4 row blocks of a KV head) takes one run, and every run of a
 // row is one more record to write and to merge. A run costs its tiles and about kSetup tiles more (the first loads and
@@ -2219,7 +2227,8 @@ void plan_own(AttnPlan& p, int n_q, int window, bool fixed_scratch) {
   // the keys a work-group's rows see, from a multiple of the tile on
   const long long range = window > 0 ? std::min<long long>(n_q, (long long)window + rows + kTile - 2) : n_q;
   const int tiles = int((range + kTile - 1) / kTile);
-  if (own_few_rows(p.d, n_q)) {
+  p.few = own_few_rows(p.d, p.group, n_q);
+  if (p.few) {
     p.own = p.own_max = 1;
     p.run = tiles * kTile;
     return;
@@ -2599,9 +2608,11 @@ std::string launch_attn_own(const AttnPlan& p, int b0, int nblocks, const float*
   a.own = p.own;
   a.run = p.run;
   a.scale2 = scale * kLog2e;
-  if (own_few_rows(p.d, n_q)) {
+  if (p.few) {
     const long long waves = (long long)p.kv_heads * (p.qpad / 16) * nblocks;
-    void (*fn)(const OwnArgs) = p.d == 128 ? attn_own_mfma_kernel<128> : attn_own_mfma_kernel<256>;
+    void (*fn)(const OwnArgs) = p.d == 64    ? attn_own_mfma_kernel<64>
+                                : p.d == 128 ? attn_own_mfma_kernel<128>
+                                             : attn_own_mfma_kernel<256>;
     hipLaunchKernelGGL(fn, dim3(unsigned((waves + 3) / 4)), dim3(256), 0, stream, a);
     HIP_CHECK(hipGetLastError());
     return strf("attn_own_mfma_kernel<%d>", p.d);

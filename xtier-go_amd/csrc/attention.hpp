@@ -52,6 +52,7 @@ struct AttnPlan {
   int tile_lo = 0, tiles = 0;  // the 32-slot tiles to scan
   int splits = 0;              // work-groups per KV head over the tiles (0: no cached key is visible)
   bool quads = false;          // the scan's work-groups take 4 row blocks each (attn_scan_rows_kernel)
+  bool few = false;            // own keys by the few-row kernel, one record
   int own = 1;                 // own-key records per (block, KV head, q-col), after the splits'
   int run = 32, window = 0;    // own keys per record, the call's window
   int own_max = 1;             // what scratch is sized for: the most records of any position in this cache,
