@@ -20,7 +20,7 @@ int main() {
                     &pos0, &window, &fixed) == 10) {
     c.ring = ring, c.fp8 = fp8, c.slots_pad = int((c.slots + 31) / 32 * 32);
     const xtg::hip::AttnPlan p = xtg::hip::attn_plan(c, n_q, heads, pos0, window, fixed != 0);
-    std::printf("%d %d %d %d %d %d %zu %zu\n", p.tiles, p.splits, int(p.quads), int(p.few), p.own, p.run, p.records() * (p.d + 2),
+    std::printf("%d %d %d %d %d %d %zu %zu\n", p.tiles, p.splits, int(p.quads), int(p.few), p.own, p.run, p.used_floats(),
                 p.part_floats());
   }
 }

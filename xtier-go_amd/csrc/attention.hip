@@ -2227,7 +2227,9 @@ void plan_own(AttnPlan& p, int n_q, int window, bool fixed_scratch) {
   // the keys a work-group's rows see, from a multiple of the tile on
   const long long range = window > 0 ? std::min<long long>(n_q, (long long)window + rows + kTile - 2) : n_q;
   const int tiles = int((range + kTile - 1) / kTile);
-  p.few = own_few_rows(p.d, p.group, n_q);
+  // (the fixed array's one run of up to kOwnChunk keys, where no more records fit: 64 / 8 heads of 128, 64 rows 16.7 us
+  // with the few-row kernel and 18.9 tiled, 100 rows 20.0 and 21.8; tiled at 256 dims 0.9 of its time)
+  p.few = own_few_rows(p.d, p.group, n_q) || (fixed_scratch && fixed == 1 && p.d != 256);
   if (p.few) {
     p.own = p.own_max = 1;
     p.run = tiles * kTile;

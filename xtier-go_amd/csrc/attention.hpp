@@ -59,6 +59,7 @@ struct AttnPlan {
   int splits_max = 0;          // whatever this call's
   int kv_heads = 1, d = 64;
   size_t records() const { return size_t(blocks) * size_t(kv_heads) * size_t(splits + own) * size_t(qpad); }
+  size_t used_floats() const { return records() * size_t(d + 2); }
   size_t part_floats() const { return records() / size_t(splits + own) * size_t(splits_max + own_max) * size_t(d + 2); }
 };
 // fixed_scratch: for the call whose partials go to the fixed array (one own-key record per kOwnChunk keys).
