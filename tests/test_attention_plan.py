@@ -82,3 +82,19 @@ def test_calls_of_few_rows_keep_the_few_row_kernel(plans, heads, kv, d, last):
     for window in (0, 1024):
         ps = plans([(kv, d, 1040, 1, 0, n, heads, 500, window, 0) for n in (9, last, last + 1)])
         assert [p.few for p in ps] == [1, 1, 0] and ps[0].own == ps[1].own == 1
+
+
+@pytest.mark.parametrize("heads,kv,d,slots,ring,ctx,n,shared", [
+    (32, 8, 128, 2100, 0, 1500, 256, 0), (32, 8, 128, 2100, 0, 1500, 320, 1), (32, 8, 128, 6600, 0, 6000, 128, 1),
+    (32, 8, 128, 1088, 1, 5000, 256, 0), (16, 4, 256, 1040, 1, 5000, 128, 0), (16, 4, 256, 1040, 1, 5000, 256, 1),
+    (2, 1, 128, 6600, 0, 6000, 384, 0), (8, 8, 128, 2100, 0, 1500, 320, 0), (8, 8, 128, 6600, 0, 6000, 512, 1),
+    (16, 8, 64, 2100, 0, 1500, 192, 0), (64, 8, 256, 2100, 0, 1500, 160, 1), (8, 1, 64, 2100, 0, 1500, 256, 0),
+    (32, 8, 128, 6600, 0, 6000, 120, 0)])
+def test_tiles_are_shared_where_that_measured_faster(plans, heads, kv, d, slots, ring, ctx, n, shared):
+    """Calls whose two scans measured at least 8 % apart (the last is below the rows that share), and the most splits a
+    work-group per CU allows."""
+    p = plans([(kv, d, slots, ring, 0, n, heads, ctx, 1024 if ring else 0, 0)])[0]
+    assert p.shared == shared
+    if shared:
+        blocks = -(-n // (32 // (heads // kv)))
+        assert p.splits <= max(1, 256 // (kv * -(-blocks // 4)))

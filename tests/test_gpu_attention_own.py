@@ -92,6 +92,18 @@ def test_many_row_scan_at_the_edges(hip, pkg, heads, kv, d, n, cached, window, r
     assert err <= 6e-5, err
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,kv,d,n,cached,window,ring", SCANS)
+def test_shared_tiles_at_the_edges(hip, pkg, monkeypatch, heads, kv, d, n, cached, window, ring, fp8):
+    """The same calls with their tiles shared, also where each block's own tiles are faster; one and several splits."""
+    monkeypatch.setenv("XTG_ATTN_SHARED", "1")
+    err = run(hip, pkg, heads, kv, d, n, cached, window, ring, fp8)
+    assert err <= 6e-5, err
+    monkeypatch.setenv("XTG_ATTN_SPLITS", "3")
+    err = run(hip, pkg, heads, kv, d, n, cached, window, ring, fp8)
+    assert err <= 6e-5, err
+
+
 def test_an_infinite_value_stays_infinite(hip):
     """A visible infinity of V gives an infinity (the split of a value into terms would make it NaN), and rows before
     its 32-row tile do not see it."""

@@ -2269,6 +2269,29 @@ void plan_own(AttnPlan& p, int n_q, int window, bool fixed_scratch) {
   }
 }
 
+// The time of a many-row call's scan in us, each row block on its own tiles or shared: rounds of work-groups over the
+// 256 CUs (own: 4 waves take a quarter of the split's tiles each; shared, below 256 dims: 2 at a time), each its tiles
+// and a set-up, and the splits' records, written and merged. Fitted to the GPU time of whole calls of 128 to 512 rows over
+// 300 to 6000 keys, 13 pairs of heads and sizes, rings and caches by position, BF16 and FP8 (546 sizes): the choice is
+// within 6 % of the faster one everywhere and costs 0.1 % on average, where taking the shared scan from 128 rows on (and
+// 32 tiles at 128 dims) cost 7.6 %, 37 % at worst. Own tiles and shared: 32 / 8 heads of 128 over 1500 keys, 256 rows 50.9
+// and 54.8 us, 320 rows (two rounds of own ones) 82.9 and 62.2; over 6000 keys, 128 rows 89.0 and 57.0; 16 / 4 of 256 over a
+// ring of 1040 FP8 slots, 128 rows 42.1 and 53.0, 256 rows 66.6 and 61.3; 2 / 1 of 128 over 6000 keys, 384 rows 38.9 and
+// 50.6.
+double scan_us(const AttnPlan& p, int heads, int n_q, int splits, bool shared) {
+  struct Cost {
+    double tile[2], setup[2], mb;   // own, shared; a MB of records
+  };
+  static constexpr Cost k64{{0.585, 0.473}, {3.48, 4.19}, 0.358}, k128{{1.446, 0.972}, {5.19, 10.8}, 0.149},
+      k256{{3.384, 2.412}, {2.57, 9.99}, 0.154};
+  const Cost& k = p.d == 64 ? k64 : p.d == 128 ? k128 : k256;
+  const int per = (p.tiles + splits - 1) / splits;
+  const int steps = !shared ? (per + kWaves - 1) / kWaves : p.d == 256 ? per : (per + 1) / 2 * 2;
+  const long long wgs = (long long)p.kv_heads * splits * (shared ? (p.blocks + kWaves - 1) / kWaves : p.blocks);
+  return double((wgs + 255) / 256) * (k.tile[shared] * steps + k.setup[shared]) +
+         k.mb * 4e-6 * double(n_q) * heads * (p.d + 2) * splits;
+}
+
 }  // namespace
 
 AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int window, bool fixed_scratch) {
@@ -2312,30 +2335,38 @@ AttnPlan attn_plan(const DevKv& c, int n_q, int heads, long long pos0, int windo
   // 8 %, and 512 work-groups take 1.5 % off the one-token step at 32K (1.099 -> 1.082 ms, with the gate's merge on
   // more waves; 0.2 % at 8K; 768 and 1024: 1.109 and 1.105 ms), while at 8 rows they cost 4 %.
   // (XTG_ATTN_SPLITS=n fixes the count, for experiments)
-  // Calls of many rows share their tiles (attn_scan_rows_kernel), a work-group per CU with at least 4 tiles each. Whole
-  // calls, each on its own tiles and shared: 64 rows over 1500 keys 29.9 and 36 us (128 dims), 47.6 and 55 us (256); 96
-  // rows 36.6 and 37.9; 128 rows 48 and 43 us, 77 and 54 us; 128 dims and few tiles, 256 rows over 300 keys, 40 and 43
-  // us, where 256 dims take 71 and 58 us. (The fixed array's calls keep the plan that fits it.)
-  auto shared = [&](int tiles) { return !fixed_scratch && n_q >= 128 && (c.head_dim != 128 || tiles >= 32); };
   const char* const env = std::getenv("XTG_ATTN_SPLITS");
-  auto splits_of = [&](int tiles) {
-    if (tiles == 0) return 0;
+  auto own_splits = [&](int tiles) {
     const int wgs = c.fp8 && !c.ring && n_q == 1 ? 512 : 192;
     const int want = std::max(1, wgs / (c.kv_heads * p.blocks));   // about wgs work-groups over all blocks
     const int mt = c.ring ? 1 : 2;
-    const int quads = c.kv_heads * ((p.blocks + kWaves - 1) / kWaves);
-    int n = env ? std::atoi(env)
-                : shared(tiles) ? std::min(256 / quads, tiles / 4)
-                                : std::min(want, (tiles + mt * kWaves - 1) / (mt * kWaves));
+    const int n = env ? std::atoi(env) : std::min(want, (tiles + mt * kWaves - 1) / (mt * kWaves));
     return std::min(std::max(1, n), tiles);
   };
-  p.splits = splits_of(p.tiles);
-  p.quads = p.tiles > 0 && shared(p.tiles);
+  p.splits = own_splits(p.tiles);
+  // Calls of many rows may share their tiles (attn_scan_rows_kernel), in at most one round of work-groups where that
+  // fits: where scan_us makes it faster. (XTG_ATTN_SHARED=0 or 1 fixes which, for experiments. The fixed array's calls keep
+  // the plan that fits it.)
+  const char* const shared = std::getenv("XTG_ATTN_SHARED");
+  const bool may_share = !fixed_scratch && (shared ? std::atoi(shared) != 0 && n_q > kProdRows : n_q >= 128);
+  const int quads = c.kv_heads * ((p.blocks + kWaves - 1) / kWaves);
+  const int most = env ? std::max(1, std::atoi(env)) : std::max(1, 256 / quads);
+  if (p.tiles > 0 && may_share) {
+    double best = shared ? INFINITY : scan_us(p, heads, n_q, p.splits, false);
+    const int first = env ? std::min(most, p.tiles) : 1;
+    for (int n = first; n <= std::max(first, std::min(most, p.tiles / 2)); ++n) {
+      const double t = scan_us(p, heads, n_q, n, true);
+      if (t >= best) continue;
+      best = t;
+      p.quads = true;
+      p.splits = n;
+    }
+  }
   // Scratch holds the most splits of any position, so that no later call of as many rows outgrows it (in the middle of a
-  // prompt, or in a graph capture): more tiles never get fewer splits, but for where tiles begin to be shared. The
-  // allocation-free call checks its own need, on a ring that of a full one.
+  // prompt, or in a graph capture). The allocation-free call checks its own need, on a ring that of a full one.
   p.splits_max = p.splits;
-  if (c.ring || !fixed_scratch) p.splits_max = std::max(splits_of(ring_tiles), splits_of(std::min(ring_tiles, 31)));
+  if (c.ring || !fixed_scratch) p.splits_max = own_splits(ring_tiles);   // more tiles never get fewer
+  if (may_share) p.splits_max = std::max(p.splits_max, std::min(most, ring_tiles));
   plan_own(p, n_q, window, fixed_scratch);
   return p;
 }
