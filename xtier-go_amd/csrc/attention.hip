@@ -2213,10 +2213,14 @@ bool own_few_rows(int d, int group, int n_q) {
 // The runs of own keys: a work-group of attn_own_kernel (4 row blocks of a KV head) takes one run, and every run of a
 // row is one more record to write and to merge. A run costs its tiles and about kSetup tiles more (the first loads and
 // record); with fewer work-groups than the chip holds at once the longest run is the launch's time, with more the
-// sum over the chip, plus half of a run at the end. A record's write and read back is counted in tiles too. The
-// candidate of the least such time is taken. Whole attention calls without cached keys, runs of 128 keys and the runs
-// taken: 188 rows, 16 / 4 heads of 256: 31.7 and 25.6 us; 256 rows of 128 dims 26 and 23 us; 512 rows, 32 / 8 heads of
-// 128: 42.2 and 37.6 us; 512 rows of 256 dims 46.3 and 48.5 us.
+// sum over the chip, plus half of a run at the end. From 192 work-groups on some CUs get two (at 256 dims: one after the
+// other) while others have none, since those without a key are dealt out among the rest. A record's write and read back
+// is counted in tiles too. The candidate of the least such time is taken. On the GPU, own keys and merge, runs of 32 keys,
+// 64, 96, 128 and 192, the one taken in brackets: 224 rows, 32 / 8 heads of 128: 26.8 [21.9] 23.8 26.6 32.5 us (by 256
+// work-groups instead of 192 it was 32 keys, slower than the FP32 kernel's 25.1); 512 rows: 55.3 46.7 [38.9] 43.1 46.8;
+// 188 rows, 16 / 4 heads of 256: [25.5] 28.3 33.1 38.4 48.8; 512 rows: 67.5 55.8 49.3 [46.3] 55.8. It is not the best
+// everywhere: over 14 pairs of heads the run taken costs 2 % on average from 64 to 512 rows (30 % at worst, 64 / 8 heads of
+// 256), and 5 % with 700 to 1500 rows (70 %), where it matters most which CUs the work-groups without a key fall on.
 // With fixed_scratch (the call that allocates nothing, whose array has a fixed size) the count is one run per
 // kOwnChunk keys, as always, so that the same calls fit.
 void plan_own(AttnPlan& p, int n_q, int window, bool fixed_scratch) {
@@ -2256,9 +2260,9 @@ void plan_own(AttnPlan& p, int n_q, int window, bool fixed_scratch) {
         wgs += n * p.kv_heads;
         work += (t + n * kSetup) * p.kv_heads;
       }
-      const double shared = slots > 256 && wgs > 256 ? 1 + 0.3 * (std::min(wgs, slots) - 256) / 256 : 1;
-      const double cost = (wgs <= slots ? rt * shared + kSetup : work / slots * shared + 0.5 * rt) +
-                          wgs * p.d * 6e-5;
+      const double crowd =
+          wgs <= 192 ? 1 : p.d == 256 ? 1.2 : 1.3 + 0.2 * std::max(0.0, std::min(wgs, slots) - 256) / 256;
+      const double cost = (wgs <= slots ? rt * crowd + kSetup : work / slots * crowd + 0.5 * rt) + wgs * p.d * 6e-5;
       if (best == 0 || cost < best * 1.01) {   // equal: the fewer records
         best = cost;
         p.own = own;
