@@ -168,20 +168,44 @@ def _ptr(a):
     return a.data_ptr()   # torch.Tensor
 
 
+class _Address(int):
+    """The address of an array, which it holds: with a second reference numpy refuses to resize (move) it in place. A copy
+    or a pickle of it reads its own array's."""
+
+    def __new__(cls, array):
+        at = int.__new__(cls, array.ctypes.data)
+        at.array = array
+        return at
+
+    def __reduce__(self):
+        return _Address, (self.array,)
+
+
 class _Array:
     """A Weight's array attribute: its address is read when the array is set, not on every call (numpy's .ctypes takes
     about 0.6 us, three times per weight of a call; a call of four projections spent half of its 14 us there)."""
 
     def __set_name__(self, owner, name):
-        self.slot = "_" + name
+        self.name, self.held = name, "_" + name
 
     def __get__(self, w, owner=None):
-        return self if w is None else getattr(w, self.slot)
+        if w is None:
+            return self
+        try:
+            return w.__dict__[self.name]
+        except KeyError:
+            raise AttributeError(self.name) from None
 
     def __set__(self, w, a):
-        setattr(w, self.slot, a)
-        setattr(w, self.slot + "_held", a)   # a second reference: numpy then refuses to resize (move) it in place
-        setattr(w, self.slot + "_at", a.ctypes.data)
+        w.__dict__[self.name] = a
+        w.__dict__.pop(self.held, None)
+        if hasattr(a, "ctypes"):
+            w.__dict__[self.held] = _Address(a)
+
+    def __delete__(self, w):
+        self.__get__(w)
+        del w.__dict__[self.name]
+        w.__dict__.pop(self.held, None)
 
 
 class Weight:
@@ -196,19 +220,11 @@ class Weight:
         self.k = self.codes.shape[1] * 2
         assert self.scales.shape == (self.n_out, self.k // 16)
 
-    def __getstate__(self):   # copies and pickles set their own arrays, and so their own addresses
-        return {"codes": self.codes, "scales": self.scales, "glob": self.glob, "n_out": self.n_out, "k": self.k}
-
-    def __setstate__(self, state):
-        for name, v in state.items():
-            setattr(self, name, v)
-
     def struct(self):
-        return Nvfp4(self._codes_at, self._scales_at, self.glob, self.n_out, self.k)
-
-
-def _structs(ws):
-    return (Nvfp4 * len(ws))(*[w.struct() for w in ws])
+        try:
+            return Nvfp4(self._codes, self._scales, self.glob, self.n_out, self.k)
+        except AttributeError:   # no addresses: restored from a state of codes and scales alone, or no arrays any more
+            return Nvfp4(self.codes.ctypes.data, self.scales.ctypes.data, self.glob, self.n_out, self.k)
 
 
 class HipBackend:
@@ -246,9 +262,10 @@ class HipBackend:
         return lib().xtg_hip_stream(self.h)
 
     def _hold(self, ws):
-        for w in ws:
-            self._weights.setdefault(w._codes_at, w)
-        return _structs(ws)
+        structs = [w.struct() for w in ws]
+        for w, st in zip(ws, structs):
+            self._weights.setdefault(st.codes, w)
+        return (Nvfp4 * len(ws))(*structs)
 
     def prepare(self, w):
         err = _errbuf()
