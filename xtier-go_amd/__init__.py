@@ -220,11 +220,15 @@ class Weight:
         self.k = self.codes.shape[1] * 2
         assert self.scales.shape == (self.n_out, self.k // 16)
 
-    def struct(self):
+    def fields(self):
+        """The values of its Nvfp4."""
         try:
-            return Nvfp4(self._codes, self._scales, self.glob, self.n_out, self.k)
+            return self._codes, self._scales, self.glob, self.n_out, self.k
         except AttributeError:   # no addresses: restored from a state of codes and scales alone, or no arrays any more
-            return Nvfp4(self.codes.ctypes.data, self.scales.ctypes.data, self.glob, self.n_out, self.k)
+            return self.codes.ctypes.data, self.scales.ctypes.data, self.glob, self.n_out, self.k
+
+    def struct(self):
+        return Nvfp4(*self.fields())
 
 
 class HipBackend:
@@ -262,10 +266,12 @@ class HipBackend:
         return lib().xtg_hip_stream(self.h)
 
     def _hold(self, ws):
-        structs = [w.struct() for w in ws]
-        for w, st in zip(ws, structs):
-            self._weights.setdefault(st.codes, w)
-        return (Nvfp4 * len(ws))(*structs)
+        arr = (Nvfp4 * len(ws))()
+        for i, w in enumerate(ws):
+            arr[i] = fields = w.fields()
+            if fields[0] not in self._weights:
+                self._weights[int(fields[0])] = w
+        return arr
 
     def prepare(self, w):
         err = _errbuf()
