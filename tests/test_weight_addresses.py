@@ -2,6 +2,7 @@
 set again, after a copy and a pickle; and numpy refuses to move an array that it holds."""
 import copy
 import pickle
+import types
 import weakref
 
 import numpy as np
@@ -45,6 +46,12 @@ def test_copies_and_pickles_keep_what_a_program_sets(pkg, monkeypatch):
     old = pkg.Weight.__new__(pkg.Weight)
     old.__dict__.update(codes=w.codes, scales=w.scales, glob=0.5, n_out=4, k=32)
     assert old.struct().codes == w.codes.ctypes.data
+    backend = types.SimpleNamespace(_weights={})
+    for ws in ([w], [other, old]):
+        arr = pkg.HipBackend._hold(backend, ws)
+        assert [(st.codes, st.scales, st.glob, st.n_out, st.k) for st in arr] == [
+            (x.codes.ctypes.data, x.scales.ctypes.data, 0.5, 4, 32) for x in ws]
+    assert backend._weights == {w.codes.ctypes.data: w, other.codes.ctypes.data: other}
 
 
 def test_arrays_can_be_let_go(pkg):

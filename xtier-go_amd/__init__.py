@@ -220,15 +220,11 @@ class Weight:
         self.k = self.codes.shape[1] * 2
         assert self.scales.shape == (self.n_out, self.k // 16)
 
-    def fields(self):
-        """The values of its Nvfp4."""
-        try:
-            return self._codes, self._scales, self.glob, self.n_out, self.k
-        except AttributeError:   # no addresses: restored from a state of codes and scales alone, or no arrays any more
-            return self.codes.ctypes.data, self.scales.ctypes.data, self.glob, self.n_out, self.k
-
     def struct(self):
-        return Nvfp4(*self.fields())
+        try:
+            return Nvfp4(self._codes, self._scales, self.glob, self.n_out, self.k)
+        except AttributeError:   # no addresses: restored from a state of codes and scales alone, or no arrays any more
+            return Nvfp4(self.codes.ctypes.data, self.scales.ctypes.data, self.glob, self.n_out, self.k)
 
 
 class HipBackend:
@@ -266,11 +262,17 @@ class HipBackend:
         return lib().xtg_hip_stream(self.h)
 
     def _hold(self, ws):
-        arr = (Nvfp4 * len(ws))()
-        for i, w in enumerate(ws):
-            arr[i] = fields = w.fields()
-            if fields[0] not in self._weights:
-                self._weights[int(fields[0])] = w
+        arr, held = (Nvfp4 * len(ws))(), self._weights
+        try:
+            for i, w in enumerate(ws):   # as Weight.struct, without a structure per weight
+                at = w._codes
+                arr[i] = at, w._scales, w.glob, w.n_out, w.k
+                if at not in held:
+                    held[int(at)] = w
+        except AttributeError:
+            for i, w in enumerate(ws):
+                arr[i] = w.struct()
+                held.setdefault(arr[i].codes, w)
         return arr
 
     def prepare(self, w):
