@@ -1250,28 +1250,39 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
       for (int u = 0; u < VU; ++u) st[u][e] = vr[16 * u * W];
     }
   };
+  // (a tile's rare case rewrites its terms, so that nothing waits for the check)
   auto put_k = [&](const float (&st)[KU][8]) {
-    const bool large = some_large(st);
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
       bf16x8 t[3];
-      if (large)
-        split_exact<true>(st[u], t);
-      else
-        split_exact<false>(st[u], t);
+      split_exact<false>(st[u], t);
 #pragma unroll
       for (int n = 0; n < 3; ++n) lk[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
+    }
+    if (some_large(st)) {
+#pragma unroll
+      for (int u = 0; u < KU; ++u) {
+        bf16x8 t[3];
+        split_exact<true>(st[u], t);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) lk[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
+      }
     }
   };
   // V that is not finite goes in as zeros and is added after the last tile: in the matrix ops it would meet the weight 0
   // of the columns that do not see its key, and make NaN of it
   bool odd = false;
   auto put_v = [&](const float (&st)[VU][8]) {
-    const bool large = some_large(st);
 #pragma unroll
     for (int u = 0; u < VU; ++u) {
       bf16x8 t[3];
-      if (large) {
+      split_exact<false>(st[u], t);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) lv[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
+    }
+    if (some_large(st)) {
+#pragma unroll
+      for (int u = 0; u < VU; ++u) {
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -1279,12 +1290,11 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
           x[e] = finite ? st[u][e] : 0.f;
           odd |= !finite;
         }
+        bf16x8 t[3];
         split_exact<true>(x, t);
-      } else {
-        split_exact<false>(st[u], t);
-      }
 #pragma unroll
-      for (int n = 0; n < 3; ++n) lv[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
+        for (int n = 0; n < 3; ++n) lv[((wave + u * W) * 3 + n) * 64 + lane] = t[n];
+      }
     }
     odd = __ballot(odd) != 0;
     if (lane == 0) odd_v[wave] = odd;
