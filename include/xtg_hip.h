@@ -173,7 +173,8 @@ typedef struct xtg_attn_args {
  * in them (for a ring: npu/xtg_npu.cpp:236-258). Queued. head_dim 64, 128 or 256, at most 8 q heads per KV head. */
 int xtg_hip_attention(xtg_hip* h, const xtg_attn_args* a, char* err, int err_len);
 /* No counterpart in the reference: xtg_hip_attention for callers that cannot allocate device memory (code under HIP
- * graph capture, tight serving loops, harnesses that forbid hipMalloc). Same arguments, kernels and results; it
+ * graph capture, tight serving loops, harnesses that forbid hipMalloc). Same arguments and kernels, and the
+ * same results wherever the other call's partials fit the array (else its own keys are summed in another order); it
  * allocates nothing: the split partials go to one fixed device array of XTG_HIP_ATTN_SCRATCH_BYTES per device, held
  * from the library's load until the process ends (profiling events are made only while xtg_hip_profile is on). A
  * call whose partials exceed the array fails (-1, the sizes in err) before anything is queued: decode and verify

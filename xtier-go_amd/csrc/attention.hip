@@ -1102,9 +1102,11 @@ __global__ void __launch_bounds__(256) attn_own_mfma_kernel(const OwnArgs a) {
 // Waves per SIMD: one at 64 and 128 dims and two work-groups a CU; at 256 dims two waves share a row block
 // (own_halves), one work-group a CU. LDS reads take half of the matrix ops' time (each operand read feeds two column
 // blocks: with one a wave they would take all of it). Measured (512 rows, no cached keys, in the kernel): 16 / 4 heads
-// of 256, 107 us with the FP32 kernel, 41 us here (38 in runs of 128 keys); 32 / 8 of 128, 51 and 28 us. The matrix ops are busy for a fifth of
+// of 256, 107 us with the FP32 kernel, 37 us here; 32 / 8 of 128, 51 and 29 us. The matrix ops are busy for a fifth of
 // that: a run is 3-4 tiles long, each 3-4 us of scores 1.1, softmax and splits 0.7, outputs 1.4 and barriers 0.8 in a
-// chain, after about 4 us of first loads and of code that is fetched the first time.
+// chain, after about 4 us of first loads and of code that is fetched the first time. Registers: all 256 are in use at
+// 128 and 256 dims, with 4 and 7 in scratch memory; of these one reload (4 registers of the query's terms at 256 dims) is
+// inside the tile loop, where it waits behind the next tile's K loads.
 
 // x = t0 + t1 + t2 exactly: each term the BF16 rounding of what is left (8 bits of the 24), so that |t1| <= 2^-8 |x|,
 // |t2| <= 2^-17 |x|, and either sign is as likely. ANY: an infinity or a NaN comes as the last term alone, which meets
@@ -1479,9 +1481,10 @@ __global__ void __launch_bounds__(kWaves* own_halves<D>() * 64, 2) attn_own_kern
 // direct loads; FP8 codes are converted to BF16 once on the way. Terms and matrix ops are the scan's: q in three terms,
 // the weights in two. On the vector ALUs, beside which the matrix ops run: no mask where a tile is seen whole, nothing
 // taken over the column's lanes but a maximum that moves, and the sums once at the end.
-// Measured, 512 rows, whole calls: 3000 BF16 keys of 32 / 8 heads of 128 121 -> 101 us (the kernel alone 98 -> 67 us,
-// 63 GFLOP of matrix ops issued: 0.95 PFLOP/s), of 16 / 4 heads of 256 141 -> 126 us; 8000 keys of 128 dims 248 -> 178
-// us; a full ring of 1040 FP8 slots of 256 dims 85 -> 66 us. Bound by the vector ALUs and the matrix ops about evenly.
+// Measured, 512 rows, whole calls, each block on its own tiles and shared: 3000 BF16 keys of 32 / 8 heads of 128 121 and 98
+// us (the kernel alone 98 and 69 us, 63 GFLOP of matrix ops issued: 0.92 PFLOP/s); 6000 keys 185 and 144 us; 6000 keys of
+// 16 / 4 heads of 256 212 and 180 us. Bound by the vector ALUs and the matrix ops about evenly. Where it is not the faster
+// one: scan_us.
 template <int D>
 constexpr int rows_key_halves() { return own_halves<D>() == 2 ? 1 : 2; }
 template <int D>

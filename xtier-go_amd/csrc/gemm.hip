@@ -20,9 +20,10 @@
 //    more slices fill the chip when rows are few: gemm_cost chooses. In LDS the four chunks of an operand column are
 //    rotated by half the column's index, so that the 16 lanes that read 16 columns at once touch every bank, while
 //    each quad of lanes still loads 64 consecutive bytes.
-//  - What bounds it, 16384 x 3072 at 512 rows (94-100 us, 1.03-1.1 PFLOP/s issued; the register-staged kernel before,
-//    112 us): timing-only copies took 62 us with the matrix ops alone (1.68 PFLOP/s; a large library f16 product
-//    reaches 1.4-1.57 here), 70 us with the LDS reads, 80 us with the dequantisation too, and the loads make it 98.
+//  - What bounds it, 16384 x 3072 at 512 rows (in the kernel 88 us, 103 GFLOP issued at 1.17 PFLOP/s; the register-staged
+//    kernel before, 112 us): timing-only copies of a form that took 98 us took 62 us with the matrix ops alone (1.68
+//    PFLOP/s; a large library f16 product reaches 1.4-1.57 here), 70 us with the LDS reads, 80 us with the
+//    dequantisation too, and the loads made the rest.
 //  - Tiles are dealt so that work-group i, which runs on XCD i mod 8, gets a contiguous run of tiles: the
 //    work-groups of one XCD share weight tiles (consecutive m-tiles of one n-tile) in that XCD's L2.
 #include <algorithm>
@@ -286,10 +287,11 @@ static GemmFn gemm_fn(const GemmShape& g, int parts) {
 // The time of a launch in a shape, in us, from a model fitted to 62 sizes (9 to 2048 rows, 1040 to 8192 inputs, 1720
 // to 16384 outputs, one and two parts) in 21 shapes: a CU's share of the work-groups runs in batches of what fits
 // it; a batch's k-tile takes the work of its work-groups (matrix ops on the SIMD's queue and KiB loaded), which a CU
-// with few waves overlaps less, or a round trip at least; adding up the K slices costs time too. The shape with the
-// least modelled time ran within 3 % of the fastest one on average (24 % at worst); with the rule before (by tile
-// counts, and the kernel before) 3072 x 4096 took 27.7 us at 37 rows, 16384 x 3072 took 119.8 us at 512 rows and
-// 2560 x 7168 in BF16 took 137.6 us at 1500 rows (whole calls), where now they take 13.9, 104 and 76 us.
+// with few waves overlaps less, or a round trip at least; adding up the K slices costs time too. Over 200 sizes (9 to
+// 2048 rows of 10 products, FP32 and BF16) the shape with the least modelled time costs 2.4 % on average over the fastest
+// one, 16 % at worst; with the rule before (by tile counts, and the kernel before) 3072 x 4096 took 27.7 us at 37 rows,
+// 16384 x 3072 took 119.8 us at 512 rows and 2560 x 7168 in BF16 took 137.6 us at 1500 rows (whole calls), where now they
+// take 12.8, 88.5 and 67.8 us.
 static double gemm_cost(const GemvCall& c, const GemmShape& g, int blocks, int kt) {
   const int mt = (blocks + g.cb - 1) / g.cb, waves = g.wn * g.ks;
   long wgs = 0;

@@ -452,7 +452,7 @@ struct WideLevel {
 };
 
 // Counts the weights w[0, n) >= floor_w whose bits >> (sh + 8) equal `prefix` (all, at the top level: sh = 20) into L,
-// from `base` up. The top level's last bucket takes everything below 2^-31.75: its mass counts as nothing. h: LDS,
+// from `base` up. The top level's last bucket takes everything below 1.25 * 2^-32: its mass counts as nothing. h: LDS,
 // 256 * 32 counters. Every thread of the work-group.
 __device__ inline void wide_count(const float* w, int n, float floor_w, int sh, uint32_t prefix, double base, WideLevel& L,
                                   unsigned long long* h) {
@@ -500,7 +500,7 @@ __device__ inline void wide_count(const float* w, int n, float floor_w, int sh, 
 
 // The first candidate (of those >= floor_w, in candidate order) at which the running sum is > r (strict) or >= r, or
 // the last one when none: its pair key, and in *at the running sum there; kPadKey when the sum crosses among weights
-// below 2^-31.75 or more than kCand weights agree in all but 4 bits. top: the row's top level, counted; sub: a level of
+// below 1.25 * 2^-32 or more than kCand weights agree in all but 4 bits. top: the row's top level, counted; sub: a level of
 // scratch; ck: LDS for kCand keys; h: LDS for 256 * 32 counters (the sort's scratch, too). Every thread.
 __device__ inline unsigned long long wide_find(const float* w, int n, float floor_w, double r, bool strict,
                                                const WideLevel& top, WideLevel& sub, unsigned long long* ck,
